@@ -1,0 +1,126 @@
+"""Products with few output tiles (gemm_rows.hip) against float64 sums of the same inputs.
+
+Bars: fp32 max_rel 2e-6 sqrt(K / 256) + 2e-6 (fp32 sums of K terms: K 2^-24 at worst, sqrt(K)
+2^-24 in practice; activations and the output add a few ulps); bf16 outputs are rounded once,
+so max_rel 2^-8 plus the fp32 part, doubled."""
+import numpy as np
+import pytest
+
+from oracle import numpy_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+F32 = np.float32
+
+
+@pytest.fixture(scope="module")
+def xp():
+    import tl_hip
+    tl_hip.ctx()
+    return tl_hip
+
+
+def bar(dt, K):
+    return 2 * 2.0 ** -8 if dt == "bf16" else 2e-6 * (K / 256) ** 0.5 + 2e-6
+
+
+def inputs(xp, dt, M, N, K, seed=0):
+    rng = np.random.default_rng(seed + M * 7 + N * 3 + K)
+    r = ref.round_bf16 if dt == "bf16" else (lambda a: a)
+    a = r(rng.standard_normal((M, K), dtype=F32))
+    w = r(rng.standard_normal((N, K), dtype=F32) / F32(K ** 0.5))
+    bias = r(rng.standard_normal(N, dtype=F32))
+    res = r(rng.standard_normal((M, N), dtype=F32))
+    return a, w, bias, res
+
+
+# (M, N, K): one row to several tiles, last tiles of one row and one column, one to many K
+# slices, K parts (the second line: too few tiles for the chip), many columns (the third)
+ROWS = [(1, 65, 128), (17, 33, 64), (24, 2304, 768), (33, 130, 192), (65, 516, 320), (129, 257, 448),
+        (24, 768, 3072), (100, 72, 4096), (300, 128, 2048), (90, 40, 8192),
+        (20, 40008, 128), (3, 32776, 192), (128, 50257, 64), (40, 33000, 128)]
+
+
+@pytest.mark.parametrize("dt", ["bf16"])
+@pytest.mark.parametrize("mnk", ROWS)
+def test_few_tiles(xp, dt, mnk):
+    M, N, K = mnk
+    a, w, bias, res = inputs(xp, dt, M, N, K)
+    da, dw, db, dres = (xp.array(t, dtype=dt) for t in (a, w, bias, res))
+    y = a.astype(np.float64) @ w.astype(np.float64).T
+    for kind in ("plain", "gelu", "residual"):
+        out = xp.empty((M, N), dt, pitch=(N + 7) // 8 * 8)
+        kw, want = {}, y
+        if kind != "plain":
+            kw, want = dict(bias=db), y + bias
+        if kind == "gelu":
+            kw["act"], want = xp.TL_ACT_GELU, ref.gelu(want).astype(np.float64)
+        if kind == "residual":
+            kw.update(residual=dres, ldr=N)
+            want = want + res
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=out, ldc=out.pitch, **kw)
+        err = ref.max_rel(out.get(), want)
+        assert err <= bar(dt, K), (dt, mnk, kind, err)
+
+
+@pytest.mark.parametrize("dt", ["bf16"])
+@pytest.mark.parametrize("cfg", [(24, 1, 4, 4, 64, 40, 37, 256), (3, 21, 8, 2, 32, 64, 5, 2048),
+                                 (40, 7, 4, 1, 64, 16, 8, 128), (5, 300, 2, 2, 64, 304, 0, 128)])
+def test_few_tiles_head_scatter(xp, dt, cfg):
+    """The QKV scatter into q and a cache at an odd position (one new position per sequence,
+    short odd prompts), with and without parts of K; untouched cache rows stay."""
+    B, T, Hq, Hkv, D, L, pos0, K = cfg
+    M, N = B * T, (Hq + 2 * Hkv) * D
+    a, w, bias, _ = inputs(xp, dt, M, N, K)
+    q, k, vt = (xp.empty(s, dt).fill(7) for s in ((B, Hq, T, D), (B, Hkv, L, D), (B, Hkv, D, L)))
+    xp.gemm(xp.array(a, dtype=dt), xp.array(w, dtype=dt), M=M, N=N, K=K, lda=K, ldb=K,
+            b_layout=xp.TL_B_NK, bias=xp.array(bias, dtype=dt),
+            qkv=(q, k, vt, T, Hq, Hkv, D, L, pos0))
+    y = (a.astype(np.float64) @ w.astype(np.float64).T + bias).reshape(B, T, Hq + 2 * Hkv, D)
+    y = y.transpose(0, 2, 1, 3)
+    kw, vw = np.full((B, Hkv, L, D), 7.0), np.full((B, Hkv, D, L), 7.0)
+    kw[:, :, pos0:pos0 + T] = y[:, Hq:Hq + Hkv]
+    vw[..., pos0:pos0 + T] = y[:, Hq + Hkv:].transpose(0, 1, 3, 2)
+    for got, want in ((q, y[:, :Hq]), (k, kw), (vt, vw)):
+        assert ref.max_rel(got.get(), want) <= bar(dt, K), cfg
+
+
+@pytest.mark.parametrize("mnk", [(24, 512, 512), (48, 1000, 4096), (100, 200, 128), (17, 66000, 64)])
+def test_few_tiles_gated(xp, mnk):
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, "bf16", M, N, K)
+    out = xp.empty((M, N // 2), "bf16")
+    xp.gemm(xp.array(a, dtype="bf16"), xp.array(w, dtype="bf16"), M=M, N=N, K=K, lda=K, ldb=K,
+            b_layout=xp.TL_B_NK, C=out, ldc=N // 2, act=xp.TL_ACT_SILU, geglu=True)
+    y = a.astype(np.float64) @ w.astype(np.float64).T
+    want = ref.silu(y[:, 0::2]).astype(np.float64) * y[:, 1::2]
+    assert ref.max_rel(out.get(), want) <= bar("bf16", K)
+
+
+@pytest.mark.parametrize("dt,mnk", [("bf16", (24, 768, 3072))])
+def test_parts_without_workspace(dt, mnk):
+    """A fresh context whose first product is captured: the workspace cannot grow then, so the
+    product takes one workgroup per tile; replays and a later eager call agree."""
+    import tl_hip as xp
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, dt, M, N, K)
+    old, xp._ctx = xp._ctx, None
+    try:
+        da, dw = xp.array(a, dtype=dt), xp.array(w, dtype=dt)
+        out = xp.empty((M, N), dt, pitch=(N + 7) // 8 * 8)
+        call = lambda: xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=out,  # noqa: E731
+                               ldc=out.pitch)
+        assert xp.ctx().workspace_bytes() == 0
+        with xp.capture() as g:
+            call()
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+        for _ in range(2):
+            g.launch()
+            assert ref.max_rel(out.get(), want) <= bar(dt, K)
+        call()
+        assert xp.ctx().workspace_bytes() > 0
+        assert ref.max_rel(out.get(), want) <= bar(dt, K)
+        g.destroy()
+    finally:
+        xp.synchronize()
+        xp._ctx = old

@@ -43,6 +43,14 @@ int workspace(tl_ctx* ctx, size_t bytes, void** ptr) {
   return TL_OK;
 }
 
+void* try_workspace(tl_ctx* ctx, size_t bytes) {
+  void* ptr = nullptr;
+  if ((ctx->capturing && bytes > ctx->ws_bytes) || workspace(ctx, bytes, &ptr) == TL_OK) return ptr;
+  (void)hipGetLastError();
+  clear_error();
+  return nullptr;
+}
+
 int enter(tl_ctx* ctx) {
   clear_error();
   if (!ctx) return fail(TL_ERR_INVALID, "null tl_ctx");

@@ -114,6 +114,9 @@ inline size_t dtype_size(int dt) {
 int enter(tl_ctx* ctx);
 // Returns the context's scratch buffer, grown to at least `bytes` (256-byte aligned).
 int workspace(tl_ctx* ctx, size_t bytes, void** ptr);
+// The same for a caller that has another way: nullptr, with no error left behind, when the
+// scratch buffer cannot be had (it would grow during a graph capture, or the device is full).
+void* try_workspace(tl_ctx* ctx, size_t bytes);
 
 // Looks up, once per device and with that device current, the address of the static scratch
 // array behind tl_attention_fwd_noalloc, stores it in ctx->noalloc_scratch, and creates
