@@ -1,4 +1,5 @@
-"""Products with few output tiles (gemm_rows.hip) against float64 sums of the same inputs.
+"""Products with few output tiles (gemm_rows.hip) and large fp32 products on the bf16 matrix
+cores (gemm_split.hip), against float64 sums of the same inputs.
 
 Bars: fp32 max_rel 2e-6 sqrt(K / 256) + 2e-6 (fp32 sums of K terms: K 2^-24 at worst, sqrt(K)
 2^-24 in practice; activations and the output add a few ulps); bf16 outputs are rounded once,
@@ -41,7 +42,7 @@ ROWS = [(1, 65, 128), (17, 33, 64), (24, 2304, 768), (33, 130, 192), (65, 516, 3
         (20, 40008, 128), (3, 32776, 192), (128, 50257, 64), (40, 33000, 128)]
 
 
-@pytest.mark.parametrize("dt", ["bf16"])
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
 @pytest.mark.parametrize("mnk", ROWS)
 def test_few_tiles(xp, dt, mnk):
     M, N, K = mnk
@@ -63,7 +64,7 @@ def test_few_tiles(xp, dt, mnk):
         assert err <= bar(dt, K), (dt, mnk, kind, err)
 
 
-@pytest.mark.parametrize("dt", ["bf16"])
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
 @pytest.mark.parametrize("cfg", [(24, 1, 4, 4, 64, 40, 37, 256), (3, 21, 8, 2, 32, 64, 5, 2048),
                                  (40, 7, 4, 1, 64, 16, 8, 128), (5, 300, 2, 2, 64, 304, 0, 128)])
 def test_few_tiles_head_scatter(xp, dt, cfg):
@@ -97,7 +98,75 @@ def test_few_tiles_gated(xp, mnk):
     assert ref.max_rel(out.get(), want) <= bar("bf16", K)
 
 
-@pytest.mark.parametrize("dt,mnk", [("bf16", (24, 768, 3072))])
+# whole tiles only, a last round split over K, everything split, tails of one row and column,
+# one K step
+SPLIT = [(2048, 2048, 256), (2305, 1025, 96), (4000, 2304, 768), (1281, 769, 3072), (1025, 2049, 32),
+         (13050, 256, 256)]
+
+
+@pytest.mark.parametrize("mnk", SPLIT)
+def test_fp32_pieces(xp, mnk):
+    M, N, K = mnk
+    a, w, bias, res = inputs(xp, "fp32", M, N, K)
+    da, dw, db, dres = (xp.array(t, dtype="fp32") for t in (a, w, bias, res))
+    y = a.astype(np.float64) @ w.astype(np.float64).T
+    out = xp.empty((M, N), "fp32", pitch=(N + 7) // 8 * 8)
+    args = dict(M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=out, ldc=out.pitch)
+    xp.gemm(da, dw, **args)
+    assert ref.max_rel(out.get(), y) <= bar("fp32", K)
+    rel = np.linalg.norm(out.get() - y) / np.linalg.norm(y)
+    assert rel <= 2.0 ** -24 * 2 * max(1.0, (K / 32) ** 0.5), rel  # 6 roundings per 32 of K
+    xp.gemm(da, dw, bias=db, residual=dres, ldr=N, **args)
+    assert ref.max_rel(out.get(), y + bias + res) <= bar("fp32", K)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
+def test_fp32_pieces_scales(xp, scale):
+    """Operands far from 1: sums as close as at scale 1 (the smallest are redone in fp32)."""
+    M, N, K = 1100, 1100, 128
+    a, w, _, _ = inputs(xp, "fp32", M, N, K)
+    a = (a * F32(scale)).astype(F32)
+    out = xp.empty((M, N), "fp32")
+    xp.gemm(xp.array(a, dtype="fp32"), xp.array(w, dtype="fp32"), M=M, N=N, K=K, lda=K, ldb=K,
+            b_layout=xp.TL_B_NK, C=out, ldc=N)
+    assert ref.max_rel(out.get(), a.astype(np.float64) @ w.astype(np.float64).T) <= bar("fp32", K)
+
+
+@pytest.mark.parametrize("mnk", [(1100, 1100, 128), (2305, 1025, 1024)])
+def test_fp32_pieces_not_finite(xp, mnk):
+    """Infinities, NaN and values past bf16's largest give what fp32 sums give, in their rows
+    and columns alone; a denormal row gives what the fp32 MFMA kernel gives."""
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, "fp32", M, N, K)
+    a[3, 5], a[70, 0], a[700, K - 1], a[900, 7] = np.inf, -np.inf, np.nan, 3.4e38
+    w[10, 9], w[600, 1] = np.inf, np.nan
+    w[20] *= F32(1e-3)  # 3.4e38 stays finite there
+    a[1000] = F32(1e-40)
+    out, old = xp.empty((M, N), "fp32"), xp.empty((M, N), "fp32")
+    for o, tile in ((out, "auto"), (old, "128x128")):  # a named tile keeps the fp32 MFMA kernel
+        xp.gemm(xp.array(a, dtype="fp32"), xp.array(w, dtype="fp32"), M=M, N=N, K=K, lda=K, ldb=K,
+                b_layout=xp.TL_B_NK, C=o, ldc=N, tile=tile)
+    got = out.get()
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+        want[np.abs(want) > 3.5e38] *= np.inf
+    far = np.abs(np.abs(want) - 3.4e38) > 1e36  # not at fp32's very edge
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want) & far
+    assert np.array_equal(got[inf], want[inf])
+    ok = np.isfinite(want) & far & np.isfinite(got)
+    assert ok.sum() >= np.isfinite(want).sum() - 4
+    rows = np.ones(M, bool)
+    rows[[900, 1000]] = False
+    assert ref.max_rel(np.where(ok, got, 0)[rows], np.where(ok, want, 0)[rows]) <= bar("fp32", K)
+    assert ref.max_rel(np.where(ok, got, 0)[900], np.where(ok, want, 0)[900]) <= bar("fp32", K)
+    with np.errstate(all="ignore"):
+        low = np.where(ok, got - old.get(), 0)[1000]
+    assert np.abs(low).max() <= K * 2.0 ** -149
+
+
+@pytest.mark.parametrize("dt,mnk", [("bf16", (24, 768, 3072)), ("fp32", (24, 768, 3072)),
+                                    ("fp32", (1281, 769, 3072))])
 def test_parts_without_workspace(dt, mnk):
     """A fresh context whose first product is captured: the workspace cannot grow then, so the
     product takes one workgroup per tile; replays and a later eager call agree."""

@@ -20,6 +20,7 @@
 
 #include "gemm_common.hpp"
 #include "gemm_rows.hpp"
+#include "gemm_split.hpp"
 
 namespace tl {
 
@@ -1485,17 +1486,28 @@ extern "C" int tl_gemm(tl_ctx* ctx, const tl_gemm_desc* d) {
   const bool mfma32_small = mfma32_layout && !mfma32 && d->K <= 1024 &&
                             ((d->M + 63) / 64) * ((d->N + 63) / 64) * batch >= 8;
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  // Products that gemm_rows.hip takes (its rule stands there): few output tiles, few rows over a
-  // stream of weights. Offsets inside a tile are 32-bit, as in the other tiled kernels.
+  // Products that gemm_rows.hip and gemm_split.hip take (their rules stand there): few output
+  // tiles, few rows over a stream of weights, and fp32 products on one or the other by modelled
+  // time. Offsets inside a tile are 32-bit, as in the other tiled kernels.
   RowsPlan rows;
-  if (mfma && d->tile == TL_TILE_AUTO && batch == 1 && !d->norm_rows && d->K % 64 == 0 &&
-      d->lda < (1 << 24) && d->ldb < (1 << 24))
-    rows = gemm_rows_plan(d->M, d->N, d->K, cus);
-  const int family = (mfma || mfma32 || mfma32_small || rows.tile >= 0) ? d->family : TL_KF_GEMM_SIMT;
+  SplitPlan split32;
+  if (d->tile == TL_TILE_AUTO && batch == 1 && !d->norm_rows && d->lda < (1 << 24) && d->ldb < (1 << 24)) {
+    if (mfma && d->K % 64 == 0) rows = gemm_rows_plan(d->M, d->N, d->K, cus);
+    if (mfma32_layout && d->K % 32 == 0) {
+      rows = gemm_rows_plan_f32(d->M, d->N, d->K, cus);
+      split32 = gemm_split_plan(d->M, d->N, d->K, cus);
+      if (rows.tile >= 0 && split32.tile >= 0) {
+        if (rows.us <= split32.us) split32.tile = -1;
+        else rows.tile = -1;
+      }
+    }
+  }
+  const int family = (mfma || mfma32 || mfma32_small || rows.tile >= 0 || split32.tile >= 0) ? d->family : TL_KF_GEMM_SIMT;
   TL_REQUIRE(family >= 0 && family < TL_KF_COUNT, "bad kernel family");
   const bool f32out = d->dtype_out == TL_F32;
   if (rows.tile >= 0)
-    return gemm_rows_launch(ctx, p, rows, f32out, family, flops, bytes);
+    return gemm_rows_launch(ctx, p, rows, d->dtype_in == TL_F32, f32out, family, flops, bytes);
+  if (split32.tile >= 0) return gemm_split_launch(ctx, p, split32, f32out, family, flops, bytes);
   const bool skinny = mfma && (d->tile == TL_TILE_SKINNY || (d->tile == TL_TILE_AUTO && d->M <= 16));
   if (d->norm_rows) {
     if (!skinny || batch != 1)

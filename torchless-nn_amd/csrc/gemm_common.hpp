@@ -1,4 +1,4 @@
-// Shared pieces of the GEMM kernels (gemm.hip, gemm_rows.hip): the parameter
+// Shared pieces of the GEMM kernels (gemm.hip, gemm_rows.hip, gemm_split.hip): the parameter
 // block, global-memory access helpers, the general epilogue and the output tile order.
 #pragma once
 

@@ -1,6 +1,7 @@
-// gemm_rows_kernel: bf16 products with too few output tiles to fill the chip on the tiles of
+// gemm_rows_kernel: products with too few output tiles to fill the chip on the tiles of
 // gemm.hip: those of a batched decode step (M = 17 .. 128 rows: a stream of the weights), of a
-// few short prompts, of a small model.
+// few short prompts, of a small model. bf16 operands on v_mfma_f32_16x16x32_bf16, fp32 ones on
+// v_mfma_f32_16x16x4f32 (as in gemm_mfma_f32_kernel).
 //
 // What bounds them is the weight stream and the start of a workgroup, not the matrix cores,
 // so a workgroup keeps whole K steps of both operands in flight on their way into LDS
@@ -194,22 +195,25 @@ __global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(GemmParams p, con
 }
 
 // The tiles, with what they cost on an MI355X: `start` us from launch to the first stage, then
-// `stage1` / `stage2` us per stage with one / two workgroups per CU. Fitted to 280 products (M = 17
-// .. 3500, N 256 .. 256000, K 256 .. 16384), each timed on 2 to 20 (tile, splits) pairs: the
-// pair that the model picks takes on average 0.8% more than the best one.
+// `stage1` / `stage2` us per stage with one / two workgroups per CU. Fitted to 280 bf16 (M = 17
+// .. 3500, N 256 .. 256000, K 256 .. 16384) and 370 fp32 products (M = 1 .. 33000, N 65 ..
+// 50257, K 128 .. 4096), each timed on 2 to 20 (tile, splits) pairs: the pair that the model
+// picks takes on average 0.8% (bf16) and 0.3% (fp32, gemm_split.hip's pairs included) more than
+// the best one. 128-column tiles stay behind the split kernel's in fp32.
 struct RowsTile {
   int bm, bn, wgk, per_cu;
   float start, stage1, stage2;
+  float start32, stage1_32, stage2_32;
 };
 static const RowsTile kRowsTiles[] = {
-    {32, 32, 4, 1, 0.3f, 0.50f, 0.60f},
-    {32, 64, 2, 2, 0.35f, 0.48f, 0.86f},
-    {64, 64, 1, 2, 0.45f, 0.25f, 0.45f},
-    {32, 128, 1, 2, 0.4f, 0.50f, 0.56f},
-    {64, 128, 1, 2, 0.5f, 0.60f, 0.72f},
-    {128, 128, 1, 2, 0.85f, 0.80f, 0.97f},
+    {32, 32, 4, 1, 0.3f, 0.50f, 0.60f, 0.2f, 0.91f, 1.0f},
+    {32, 64, 2, 2, 0.35f, 0.48f, 0.86f, 0.35f, 0.9f, 1.3f},
+    {64, 64, 1, 2, 0.45f, 0.25f, 0.45f, 0.4f, 0.55f, 1.08f},
+    {32, 128, 1, 2, 0.4f, 0.50f, 0.56f, 0, 0, 0},
+    {64, 128, 1, 2, 0.5f, 0.60f, 0.72f, 0, 0, 0},
+    {128, 128, 1, 2, 0.85f, 0.80f, 0.97f, 0, 0, 0},
 };
-constexpr int kNumRowsTiles = sizeof(kRowsTiles) / sizeof(kRowsTiles[0]);
+constexpr int kNumRowsTiles = sizeof(kRowsTiles) / sizeof(kRowsTiles[0]), kNumRowsTiles32 = 3;
 
 template <typename TI, typename TO>
 static void launch_rows(int tile, dim3 grid, hipStream_t st, const GemmParams& p, float* part, int s) {
@@ -230,11 +234,12 @@ static void launch_rows(int tile, dim3 grid, hipStream_t st, const GemmParams& p
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Modelled time (us, without what all choices share) of `splits` K ranges on one tile.
-static float rows_cost(const RowsTile& t, int64_t M, int64_t N, int64_t nslices, int splits, int cus) {
+static float rows_cost(const RowsTile& t, int64_t M, int64_t N, int64_t nslices, int splits, int elem,
+                       int cus) {
   const int64_t wgs = ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
   const float stages = (float)ceil_div(ceil_div(nslices, splits), t.wgk);
-  const float one = t.start + stages * t.stage1;
-  const float two = t.start + stages * t.stage2;
+  const float one = elem == 2 ? t.start + stages * t.stage1 : t.start32 + stages * t.stage1_32;
+  const float two = elem == 2 ? t.start + stages * t.stage2 : t.start32 + stages * t.stage2_32;
   const int64_t slots = (int64_t)t.per_cu * cus, full = wgs / slots, rest = wgs % slots;
   float us = full * (t.per_cu == 1 ? one : two);
   if (rest) us += rest <= cus ? one : two;
@@ -243,11 +248,11 @@ static float rows_cost(const RowsTile& t, int64_t M, int64_t N, int64_t nslices,
   return us;
 }
 
-// The cheapest pair.
-static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int cus) {
+// The cheapest pair among the first `ntiles` tiles.
+static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int elem, int ntiles, int cus) {
   RowsPlan best;
-  const int64_t nslices = K / 64;
-  for (int i = 0; i < kNumRowsTiles; ++i) {
+  const int64_t nslices = K / (128 / elem);
+  for (int i = 0; i < ntiles; ++i) {
     const RowsTile& t = kRowsTiles[i];
     if (t.bm > 32 && t.bm >= 2 * M) continue;  // half padding
     const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
@@ -255,7 +260,7 @@ static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int cus) {
     for (int s = 1; s <= 16; ++s) {
       // each part keeps at least three slices, and the parts fit two rounds of the chip
       if (s > 1 && (nslices / s < 3 || tiles * s > 4LL * cus)) break;
-      const float us = rows_cost(t, M, N, nslices, s, cus);
+      const float us = rows_cost(t, M, N, nslices, s, elem, cus);
       if (best.tile < 0 || us < best.us) {
         best.tile = i;
         best.splits = s;
@@ -270,7 +275,7 @@ RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
   // M <= 16: the weight-streaming kernels of gemm.hip start faster (3 to 30% on K <= 2048), but
   // read less of a wide weight at a time: 4 x 50257 x 768 21.5 us against 18.2 here, 4 x 256000
   // x 2048 212 against 178, 4 x 32768 x 2048 34.4 against 32.5, 4 x 8192 x 1024 equal.
-  if (M <= 16) return N >= 32768 ? rows_best(M, N, K, cus) : RowsPlan();
+  if (M <= 16) return N >= 32768 ? rows_best(M, N, K, 2, kNumRowsTiles, cus) : RowsPlan();
   // Products that fill the chip on the tiles of gemm.hip stay there (at 2331 x 2304 x 768 14.9
   // us against 18.8 here), with two exceptions. M <= 64, or <= 128 over many columns, is a
   // stream of the weights, and 256-row tiles only load padding with it (48 x 32768 x 2048 42.4
@@ -286,7 +291,11 @@ RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
   const bool stream = M <= 64 || (M <= 128 && t128 * 2 >= 3LL * cus);
   const bool long_k = K >= 4096 && t128 * 4 <= 5LL * cus;
   if (fills && !stream && !long_k) return RowsPlan();
-  return rows_best(M, N, K, cus);
+  return rows_best(M, N, K, 2, kNumRowsTiles, cus);
+}
+
+RowsPlan gemm_rows_plan_f32(int64_t M, int64_t N, int64_t K, int cus) {
+  return rows_best(M, N, K, 4, kNumRowsTiles32, cus);
 }
 
 template <typename TI, typename TO>
@@ -299,7 +308,7 @@ static void launch_rows_all(const RowsPlan& plan, dim3 grid, hipStream_t st, con
   }
 }
 
-int gemm_rows_launch(tl_ctx* ctx, GemmParams p, RowsPlan plan, bool f32out, int family,
+int gemm_rows_launch(tl_ctx* ctx, GemmParams p, RowsPlan plan, bool f32in, bool f32out, int family,
                      double flops, double bytes) {
   const RowsTile& t = kRowsTiles[plan.tile];
   p.tiles_m = (int)((p.M + t.bm - 1) / t.bm);
@@ -312,7 +321,9 @@ int gemm_rows_launch(tl_ctx* ctx, GemmParams p, RowsPlan plan, bool f32out, int 
   }
   const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * plan.splits));
   LaunchScope ls(ctx, family, flops, bytes);
-  if (f32out) launch_rows_all<bf16_t, float>(plan, grid, ctx->stream, p, part, ld);
+  if (f32in && f32out) launch_rows_all<float, float>(plan, grid, ctx->stream, p, part, ld);
+  else if (f32in) launch_rows_all<float, bf16_t>(plan, grid, ctx->stream, p, part, ld);
+  else if (f32out) launch_rows_all<bf16_t, float>(plan, grid, ctx->stream, p, part, ld);
   else launch_rows_all<bf16_t, bf16_t>(plan, grid, ctx->stream, p, part, ld);
   return ls.finish("gemm_rows");
 }

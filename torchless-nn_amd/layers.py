@@ -14,8 +14,8 @@ reference; every forward is a handful of libtl kernel launches on one HIP stream
 The MFMA GEMMs read a weight in a K-contiguous copy ([out, in]) that is packed on the
 device the first time the weight is used and again after its buffer has been written (by
 `set`, `fill` or any kernel writing into any view of it). bf16 weights always take that copy;
-fp32 weights take it for products the fp32 matrix-core kernels run (K % 4 == 0, and either
-at least 128 output tiles of 128x128 or K <= 1024 with at least 8 tiles of 64x64), which
+fp32 weights take it for products the matrix-core kernels run (K % 32 == 0; or K % 4 == 0 and
+either at least 128 output tiles of 128x128 or K <= 1024 with at least 8 tiles of 64x64), which
 doubles their HBM use, and are read in place by the fp32 VALU GEMM otherwise.
 """
 import numpy as np
@@ -101,11 +101,15 @@ def linear(x2d, w, bias=None, act=xp.TL_ACT_NONE, residual=None, out=None, qkv=N
     x2d, norm_eps = _prenorm(x2d, prenorm, w.dtype)
     if qkv is None and out is None:
         out = xp.empty((M, N), x2d.dtype)
-    # bf16 always; fp32 when the fp32 matrix-core kernels take the product (K % 4 == 0, and
-    # either at least 128 output tiles of 128x128 or K <= 1024 with 8 or more 64x64 tiles):
-    # both read B as [N, K]
+    # bf16 always; fp32 when a matrix-core kernel takes the product, which reads B as [N, K]:
+    # K % 4 == 0 and either at least 128 output tiles of 128x128 or K <= 1024 with 8 or more
+    # 64x64 tiles, or any other K % 32 == 0 (24 x 768 x 3072: 37 us on the vector ALUs, 14 us
+    # packed). A weight not packed yet is not packed for the last kind inside a graph capture,
+    # where the copy would be recorded instead of made.
     if w.dtype is xp.bfloat16 or (K % 4 == 0 and (-(-M // 128) * -(-N // 128) >= 128 or
-                                                  (K <= 1024 and -(-M // 64) * -(-N // 64) >= 8))):
+                                                  (K <= 1024 and -(-M // 64) * -(-N // 64) >= 8))) or (
+            K % 32 == 0 and w.dtype is xp.float32 and
+            (not xp.capturing() or (w._aux is not None and w._aux[0] == (w._version,)))):
         B, ldb, layout = _packed_nk(w, fold), K, xp.TL_B_NK
     else:
         B, ldb, layout = w, w.pitch, xp.TL_B_KN

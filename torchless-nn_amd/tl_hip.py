@@ -256,6 +256,7 @@ class Context:
         self.handle = h
         self.device = device
         self.lib = lib
+        self.capturing = False  # between tl_graph_begin and tl_graph_end
 
     def sync(self):
         check(self.lib.tl_sync(self.handle))
@@ -1054,12 +1055,14 @@ class capture:  # noqa: N801  (used as a context manager, like torch.cuda.graph)
     def __enter__(self):
         c = ctx()
         check(c.lib.tl_graph_begin(c.handle))
+        c.capturing = True
         self.graph = None
         return self
 
     def __exit__(self, exc_type, exc, tb):
         c = ctx()
         h = ctypes.c_void_p()
+        c.capturing = False
         rc = c.lib.tl_graph_end(c.handle, ctypes.byref(h))
         if exc_type is None:
             check(rc)
@@ -1074,6 +1077,11 @@ class capture:  # noqa: N801  (used as a context manager, like torch.cuda.graph)
     def destroy(self):
         if self.graph is not None:
             self.graph.destroy()
+
+
+def capturing() -> bool:
+    """Whether the context stream is being captured into a graph."""
+    return ctx().capturing
 
 
 def attention_supported(dtype, head_dim, kv_capacity) -> bool:
