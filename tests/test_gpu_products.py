@@ -193,3 +193,68 @@ def test_parts_without_workspace(dt, mnk):
     finally:
         xp.synchronize()
         xp._ctx = old
+
+
+def attention_exact(q, k, vt, causal, offset, Tk):
+    """float64 attention of q [B, H, T, D] over the first Tk keys, heads merged [B, T, H D]."""
+    q, k, v = (t.astype(np.float64) for t in (q, k[:, :, :Tk], np.swapaxes(vt[..., :Tk], 2, 3)))
+    g = q.shape[1] // k.shape[1]
+    k, v = np.repeat(k, g, 1), np.repeat(v, g, 1)
+    s = q @ np.swapaxes(k, 2, 3) / q.shape[-1] ** 0.5
+    if causal:
+        T = q.shape[2]
+        s = np.where(np.arange(Tk)[None] <= np.arange(T)[:, None] + offset, s, -np.inf)
+    e = np.exp(s - s.max(-1, keepdims=True))
+    y = (e / e.sum(-1, keepdims=True)) @ v
+    return y.transpose(0, 2, 1, 3).reshape(q.shape[0], q.shape[2], -1)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("case", [(1, 4, 2, 65, 97, 104, True, 32), (2, 2, 2, 130, 130, 136, False, 0),
+                                  (1, 4, 1, 1, 300, 304, True, 299), (3, 2, 1, 33, 129, 136, True, 96),
+                                  (1, 2, 2, 97, 193, 200, False, 0), (2, 3, 3, 321, 321, 328, True, 0)])
+def test_fp32_attention_pieces(xp, D, case):
+    """Row blocks and key halves with remainders, grouped heads, a cache whose padding holds NaN,
+    masked halves. Probabilities sum to 1, so errors are a few fp32 ulps of the values."""
+    B, Hq, Hkv, T, Tk, L, causal, off = case
+    rng = np.random.default_rng(T + Tk + D)
+    q = rng.standard_normal((B, Hq, T, D), dtype=F32) * 2
+    k, vt = (rng.standard_normal(s, dtype=F32) for s in ((B, Hkv, L, D), (B, Hkv, D, L)))
+    k[:, :, Tk:], vt[..., Tk:] = np.nan, np.nan
+    out = xp.empty((B, T, Hq * D), "fp32")
+    xp.attention(*(xp.array(t, dtype="fp32") for t in (q, k, vt)), out, n_heads_q=Hq, n_heads_kv=Hkv,
+                 divisor=float(F32(D ** 0.5)), causal=causal, offset=off, seq_k=Tk)
+    assert ref.max_rel(out.get(), attention_exact(q, k, vt, causal, off, Tk)) <= 4e-6
+
+
+@pytest.mark.parametrize("D", [32, 64])
+def test_fp32_attention_pieces_not_finite(xp, D):
+    """Rows that see an infinite score or value, a NaN, or only tiny values give what float64
+    gives; a key with score -inf drops out."""
+    B, H, T = 1, 2, 200
+    rng = np.random.default_rng(D)
+    q, k = (rng.standard_normal((B, H, T, D), dtype=F32) for _ in range(2))
+    vt = rng.standard_normal((B, H, D, T), dtype=F32)
+    q[..., 0] = np.abs(q[..., 0]) + F32(0.1)
+    k[0, 0, 40, 0] = -np.inf         # head 0: key 40 drops out of every later row
+    vt[0, 0, 3, 150] = np.inf        # and value 150 is infinite in one dimension
+    vt[0, 0, 4, 180] = np.nan
+    vt[0, 1] *= F32(1e-33)           # head 1: pieces of the values underflow
+    out = xp.empty((B, T, H * D), "fp32")
+    xp.attention(*(xp.array(t, dtype="fp32") for t in (q, k, vt)), out, n_heads_q=H, n_heads_kv=H,
+                 divisor=float(F32(D ** 0.5)), causal=True, offset=0, seq_k=T)
+    with np.errstate(all="ignore"):
+        want = attention_exact(q, np.where(np.isinf(k), -1e300, k.astype(np.float64)), vt, True, 0, T)
+    # probabilities of masked keys are 0, and 0 * inf is NaN in the oracle and within a 16-row
+    # tile of the kernel: rows before the infinite and the NaN value's tiles never see them
+    got = out.get()
+    clean = vt.copy()
+    clean[~np.isfinite(clean)] = 0
+    low = attention_exact(q, np.where(np.isinf(k), -1e300, k.astype(np.float64)), clean, True, 0, T)
+    want[:, :144, 3], want[:, :176, 4] = low[:, :144, 3], low[:, :176, 4]
+    assert np.array_equal(np.isnan(got[0, 180:, 4]), np.isnan(want[0, 180:, 4]))
+    assert np.all(np.isposinf(got[0, 150:, 3]))
+    for cols in (slice(0, 3), slice(5, D), slice(D, 2 * D)):
+        assert ref.max_rel(got[..., cols], want[..., cols]) <= 4e-6, cols
+    assert ref.max_rel(got[0, :144, 3], want[0, :144, 3]) <= 4e-6
+    assert ref.max_rel(got[0, :176, 4], want[0, :176, 4]) <= 4e-6

@@ -18,6 +18,7 @@
 // The final O / l is written as 4 consecutive head-dim values per lane.
 #include <mutex>
 
+#include "fp32_pieces.hpp"
 #include "tl_internal.hpp"
 
 namespace tl {
@@ -1301,6 +1302,341 @@ __global__ __launch_bounds__(256) void attention_fwd_f32_kernel(AttnParams p) {
   }
 }
 
+// attention_fwd_pieces_kernel: fp32 attention (head dims 32 and 64) on the bf16 matrix cores, every
+// product taken as six products of bf16 pieces (fp32_pieces.hpp): scores, probabilities and sums
+// keep fp32 precision, with 16 MFMA cycles where the fp32 MFMA takes 43.
+//
+// A workgroup of 4 waves takes 64 query rows of one head and walks the keys in chunks of 64. Wave
+// (rg, kh) owns 32 rows (two 16-row tiles, so that a K or V^T fragment read from LDS serves twice:
+// with 16 rows per wave the fragment reads would take as long as the MFMAs) and half kh of each
+// chunk's keys, with its own running maximum and sum; the halves' results are merged at the end.
+// The chunk's K and V^T elements go through registers, are split there, and are stored as three
+// bf16 planes each (one 48 KB buffer at head dim 64: three workgroups per CU, whose loads,
+// splitting and MFMAs overlap each other's). Heavy causal blocks are dispatched first.
+//
+// A wave whose merged outputs are not all finite, or tiny, redoes its 32 rows with the fp32 MFMA
+// straight from memory (attend_rows_f32), so infinities, NaN and tiny operands give what fp32 sums
+// give.
+//
+// GPT-2-small heads, 4 x 1000 tokens: 110 -> 63 us (98 TFLOP/s of fp32 products); 8 x 1024: 150 ->
+// 104; error against 64 bits 2.0e-7 (fp32 MFMA 3.3e-7). Bound by issue: the splitting and the
+// softmax take as many cycles as the MFMAs, at two waves per SIMD (213 registers). Held to 168 for
+// three it spills and took 80 us, without the register prefetch 70; more independent sums between
+// two products of one changed nothing.
+template <int D>
+__device__ __forceinline__ void attend_rows_f32(const AttnParams& p, const float* qh, const float* kh,
+                                             const float* vh, float* oh, int row0) {
+  constexpr int DT = D / 16;
+  const int lane = threadIdx.x & 63, fr = lane & 15, fg = lane >> 4;
+  const int qpos = row0 + fr;
+  const float* qrow = qh + (int64_t)min(qpos, p.Tq - 1) * D + fg;
+  int kv_end = p.Tk;
+  if (p.causal) kv_end = (int)min((int64_t)p.Tk, (int64_t)min(row0 + 15, p.Tq - 1) + p.offset + 1);
+  f32x4 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_part = 0.f;
+#pragma unroll 1
+  for (int kv0 = 0; kv0 < kv_end; kv0 += 16) {
+    const float* krow = kh + (int64_t)min(kv0 + fr, p.Tk - 1) * D + fg;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int d = 0; d < D; d += 4) s = __builtin_amdgcn_mfma_f32_16x16x4f32(krow[d], qrow[d], s, 0, 0, 0);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int key = kv0 + 4 * fg + v;
+      s[v] = key < p.Tk && (!p.causal || key <= (int64_t)qpos + p.offset) ? s[v] : -INFINITY;
+      mx = fmaxf(mx, s[v]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx * p.scale_log2);
+    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
+    m_run = m_new;
+    l_part *= alpha;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[t][v] *= alpha;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      s[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], p.scale_log2, -m_ref));
+      l_part += s[v];
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const float* vrow = vh + (int64_t)(16 * t + fr) * p.Lk;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int key = kv0 + 4 * fg + v;
+        const float x = vrow[min(key, p.Tk - 1)];
+        o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(key < p.Tk ? x : 0.f, s[v], o[t], 0, 0, 0);
+      }
+    }
+  }
+  float l = l_part + __shfl_xor(l_part, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (qpos >= p.Tq) return;
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+    *reinterpret_cast<f32x4*>(oh + (int64_t)qpos * p.ld_out + 16 * t + 4 * fg) =
+        f32x4{o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv};
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p, int n_bh) {
+  constexpr int BKV = 64, KS = D / 32, DT = D / 16, KCH = D / 8;
+  constexpr int KU = BKV * KCH / 256, VU = D * 8 / 256;  // 8-element units per thread: K, V^T
+  constexpr int KPL = BKV * D, VPL = D * BKV;            // elements of a plane
+  static_assert(D == 32 || D == 64, "head dims 32 and 64");
+  __shared__ __attribute__((aligned(16))) bf16_t S[3 * KPL + 3 * VPL];
+  bf16_t* Ks = S;
+  bf16_t* Vs = S + 3 * KPL;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rg = wave & 1, kh2 = wave >> 1;  // row group, half of each chunk's keys
+  const int fr = lane & 15, fg = lane >> 4;
+  const int rank = (int)blockIdx.x / n_bh, bh = (int)blockIdx.x - rank * n_bh;
+  const int b = bh / p.Hq, h = bh - b * p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int nqb = (p.Tq + 63) / 64, qb = p.causal ? nqb - 1 - rank : rank;
+  const int q0 = qb * 64 + rg * 32;
+  const float* qh = reinterpret_cast<const float*>(p.q) + (int64_t)bh * p.Tq * D;
+  const float* kh = reinterpret_cast<const float*>(p.k) + (int64_t)(b * p.Hkv + hk) * p.Lk * D;
+  const float* vh = reinterpret_cast<const float*>(p.vt) + (int64_t)(b * p.Hkv + hk) * D * p.Lk;
+  float* oh = reinterpret_cast<float*>(p.out) + (int64_t)b * p.Tq * p.ld_out + (int64_t)h * D;
+
+  int kv_end = p.Tk;
+  if (p.causal) kv_end = (int)min((int64_t)p.Tk, (int64_t)min(qb * 64 + 63, p.Tq - 1) + p.offset + 1);
+  const int nchunks = (kv_end + BKV - 1) / BKV;
+
+  // unit u of a chunk: K row u / KCH, elements 8 (u % KCH) ..; V^T row u / 8, keys 8 (u % 8) ..
+  float rk[KU][8], rv[VU][8];
+  auto load_chunk = [&](int kv0) {
+#pragma unroll
+    for (int i = 0; i < KU; ++i) {
+      const int u = i * 256 + tid, kv = kv0 + u / KCH;
+      const float* src = kh + (int64_t)min(kv, p.Tk - 1) * D + 8 * (u % KCH);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(src), y = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        rk[i][e] = x[e];
+        rk[i][4 + e] = y[e];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < VU; ++i) {
+      const int u = i * 256 + tid, kv = kv0 + 8 * (u & 7);
+      const float* src = vh + (int64_t)(u >> 3) * p.Lk + min(kv, p.Lk - 8);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(src), y = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        rv[i][e] = x[e];
+        rv[i][4 + e] = y[e];
+      }
+    }
+  };
+  auto kslot = [&](int r, int c) {  // 16-byte chunk c of a K row, swizzled
+    return r * D + ((c ^ (KCH == 8 ? r & 7 : (r >> 1) & 3)) << 3);
+  };
+  auto store_chunk = [&](int kv0) {
+    if (kv0 + BKV > p.Tk) {  // values past Tk (never written) are zeroed: 0 * NaN is not 0
+#pragma unroll
+      for (int i = 0; i < VU; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          rv[i][e] = kv0 + 8 * ((i * 256 + tid) & 7) + e < p.Tk ? rv[i][e] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < KU; ++i) {
+      const int u = i * 256 + tid;
+      uint4 a, b2, c;
+      split8(rk[i], a, b2, c);
+      bf16_t* dst = Ks + kslot(u / KCH, u % KCH);
+      *reinterpret_cast<uint4*>(dst) = a;
+      *reinterpret_cast<uint4*>(dst + KPL) = b2;
+      *reinterpret_cast<uint4*>(dst + 2 * KPL) = c;
+    }
+#pragma unroll
+    for (int i = 0; i < VU; ++i) {  // two 4-key groups, in the key order of the P.V operand
+      const int u = i * 256 + tid, r = u >> 3, g = 2 * (u & 7);
+      uint4 a, b2, c;
+      split8(rv[i], a, b2, c);
+      bf16_t* lo = Vs + r * BKV + vperm_slot(g, r);
+      bf16_t* hi = Vs + r * BKV + vperm_slot(g + 1, r);
+      *reinterpret_cast<uint2*>(lo) = make_uint2(a.x, a.y);
+      *reinterpret_cast<uint2*>(hi) = make_uint2(a.z, a.w);
+      *reinterpret_cast<uint2*>(lo + VPL) = make_uint2(b2.x, b2.y);
+      *reinterpret_cast<uint2*>(hi + VPL) = make_uint2(b2.z, b2.w);
+      *reinterpret_cast<uint2*>(lo + 2 * VPL) = make_uint2(c.x, c.y);
+      *reinterpret_cast<uint2*>(hi + 2 * VPL) = make_uint2(c.z, c.w);
+    }
+  };
+
+  load_chunk(0);
+  // query pieces: lane holds Q[q0 + 16 rt + fr][32 ks + 8 fg ..]
+  bf16x8 qf[2][KS][3];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const float* qrow = qh + (int64_t)min(q0 + 16 * rt + fr, p.Tq - 1) * D + 8 * fg;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = qrow[32 * ks + e];
+      uint4 a, b2, c;
+      split8(x, a, b2, c);
+      qf[rt][ks][0] = __builtin_bit_cast(bf16x8, a);
+      qf[rt][ks][1] = __builtin_bit_cast(bf16x8, b2);
+      qf[rt][ks][2] = __builtin_bit_cast(bf16x8, c);
+    }
+  }
+  f32x4 o[2][DT];
+  float m_run[2], l_part[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    m_run[rt] = -INFINITY;
+    l_part[rt] = 0.f;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  for (int ch = 0; ch < nchunks; ++ch) {
+    if (ch) __syncthreads();  // every wave has read the chunk before
+    store_chunk(ch * BKV);
+    if (ch + 1 < nchunks) load_chunk((ch + 1) * BKV);
+    __syncthreads();
+    const int kv0 = ch * BKV + 32 * kh2;  // this wave's 32 keys
+    // none of them visible to any of its rows: nothing to add
+    if (kv0 >= p.Tk || (p.causal && kv0 > (int64_t)(q0 + 31) + p.offset)) continue;
+    f32x4 s[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 32 * kh2 + 16 * j + fr;
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) s[rt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16_t* src = Ks + kslot(r, 4 * ks + fg);
+        bf16x8 kf[3];
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) kf[pl] = *reinterpret_cast<const bf16x8*>(src + pl * KPL);
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt)
+            s[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kPieceA[t]], qf[rt][ks][kPieceB[t]], s[rt][j], 0, 0, 0);
+      }
+    }
+    const bool full = kv0 + 32 <= p.Tk && (!p.causal || (int64_t)(kv0 + 31) <= (int64_t)q0 + p.offset);
+    bf16x8 pf[2][3];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      float mx = -INFINITY;
+      if (!full) {
+        // key kv0 + 16 j + 4 fg + v is visible when 16 j + v <= lim (one per-lane limit)
+        const int lim = (int)max(min((int64_t)p.Tk - 1, p.causal ? (int64_t)(q0 + 16 * rt + fr) + p.offset
+                                                                 : (int64_t)p.Tk - 1) - kv0 - 4 * fg, (int64_t)-1);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) s[rt][j][v] = 16 * j + v <= lim ? s[rt][j][v] : -INFINITY;
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) mx = fmaxf(mx, s[rt][j][v]);
+      if (__any(mx * p.scale_log2 > m_run[rt] + 8.0f)) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float mxs = mx * p.scale_log2;
+        const float m_new = mxs > m_run[rt] + 8.0f ? mxs : m_run[rt];
+        const float alpha = __builtin_amdgcn_exp2f(m_run[rt] - m_new);
+        l_part[rt] *= m_new == -INFINITY ? 1.f : alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) o[rt][t][v] *= m_new == -INFINITY ? 1.f : alpha;
+        m_run[rt] = m_new;
+      }
+      const float m_ref = m_run[rt] == -INFINITY ? 0.f : m_run[rt];
+      float e[8];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          e[4 * j + v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[rt][j][v], p.scale_log2, -m_ref));
+          l_part[rt] += e[4 * j + v];
+        }
+      uint4 a, b2, c;
+      split8(e, a, b2, c);
+      pf[rt][0] = __builtin_bit_cast(bf16x8, a);
+      pf[rt][1] = __builtin_bit_cast(bf16x8, b2);
+      pf[rt][2] = __builtin_bit_cast(bf16x8, c);
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const int r = 16 * t + fr;
+      const bf16_t* src = Vs + r * BKV + vperm_piece(kh2, fg, r);
+      bf16x8 vf[3];
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) vf[pl] = *reinterpret_cast<const bf16x8*>(src + pl * VPL);
+#pragma unroll
+      for (int u = 0; u < 6; ++u)
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+          o[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kPieceA[u]], pf[rt][kPieceB[u]], o[rt][t], 0, 0, 0);
+    }
+  }
+
+  // merge the two key halves of each row group: the second leaves its state in LDS
+  float* red = reinterpret_cast<float*>(S) + rg * (2 * (DT * 4 + 2) * 64) + lane;
+  static_assert(2 * 2 * (DT * 4 + 2) * 64 * 4 <= (int)sizeof(S), "merge space");
+  __syncthreads();
+  if (kh2 == 1) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      float* w = red + rt * (DT * 4 + 2) * 64;
+      w[0] = m_run[rt];
+      w[64] = l_part[rt];
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) w[(2 + 4 * t + v) * 64] = o[rt][t][v];
+    }
+  }
+  __syncthreads();
+  if (kh2 == 1) return;
+  bool bad = false;
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const float* w = red + rt * (DT * 4 + 2) * 64;
+    const float m2 = w[0], m = fmaxf(m_run[rt], m2), m_ref = m == -INFINITY ? 0.f : m;
+    const float f1 = __builtin_amdgcn_exp2f(m_run[rt] - m_ref), f2 = __builtin_amdgcn_exp2f(m2 - m_ref);
+    float l = l_part[rt] * f1 + w[64] * f2;
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const float inv = 1.0f / l;
+    const int qpos = q0 + 16 * rt + fr;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      f32x4 y;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        y[v] = (o[rt][t][v] * f1 + w[(2 + 4 * t + v) * 64] * f2) * inv;
+        bad = bad || pieces_doubtful(y[v]);
+      }
+      if (qpos < p.Tq) *reinterpret_cast<f32x4*>(oh + (int64_t)qpos * p.ld_out + 16 * t + 4 * fg) = y;
+    }
+  }
+  if (__any(bad)) {
+#pragma unroll 1
+    for (int r = 0; r < 32; r += 16) attend_rows_f32<D>(p, qh, kh, vh, oh, q0 + r);
+  }
+}
+
 // Decode split: waves per workgroup and 16-key tiles per wave. 2 waves x 32 keys was the
 // fastest on an MI355X at the config-5 decode shape (B = 4, 2176 keys, D = 256) against
 // (4, 4), (1, 4), (1, 2), (4, 2) and (2, 4): 12.0 us per layer with the combine, 13.5 us
@@ -1382,6 +1718,17 @@ static int attention_fwd(tl_ctx* ctx, const void* q, const void* k, const void* 
                  dtype == TL_F32 ? 2.0 * bytes : bytes);
   if (dtype == TL_F32) {
     const int64_t nqb = (seq_q + 63) / 64;
+    // bf16 pieces on the bf16 matrix cores beyond 96 keys; for fewer the fp32 MFMA's shorter set-up
+    // is as fast or faster (us, fp32 / pieces: T = 17 7.0 / 10.5, 64 9.3 / 10.9, 65 32.2 / 34.4,
+    // 80 15.1 / 12.9, 96 14.9 / 12.7 and 18.9 / 19.5, 128 11.6 / 9.2, 150 29 / 25, 261 69 / 48,
+    // 1000 110 / 63, 1 query on 900 keys 87 / 57)
+    if (head_dim <= 64 && seq_k > 96 && nqb * batch * n_heads_q < (1LL << 31)) {
+      const int n_bh = (int)(batch * n_heads_q);
+      const dim3 g((unsigned)(nqb * n_bh));
+      if (head_dim == 32) attention_fwd_pieces_kernel<32><<<g, 256, 0, ctx->stream>>>(p, n_bh);
+      else attention_fwd_pieces_kernel<64><<<g, 256, 0, ctx->stream>>>(p, n_bh);
+      return ls.finish("attention_fwd_pieces");
+    }
     const dim3 grid((unsigned)(causal ? (nqb + 1) / 2 : nqb), (unsigned)(batch * n_heads_q));
     switch (head_dim) {
       case 32: attention_fwd_f32_kernel<32, 32><<<grid, 256, 0, ctx->stream>>>(p); break;

@@ -2,13 +2,9 @@
 // TFLOP/s, the bf16 one at 2.5 PFLOP/s, so six bf16 products per fp32 product have 2.6 times
 // the room.
 //
-// Every operand element is split into three bf16 pieces x = x1 + x2 + x3, each the rounding of
-// what the pieces before it leave (8 + 8 + 8 significand bits and the signs cover fp32's 24, so
-// the split is exact while x3 is representable, |x| >= 2^-110), and
-//   a b = a1 b1 + (a1 b2 + a2 b1) + (a1 b3 + a2 b2 + a3 b1) + O(2^-24 a b):
-// the three products left out are below half an fp32 ulp of a b. The bf16 products are exact and
-// accumulate in fp32 like the fp32 MFMA's, with fewer roundings (6 accumulating instructions per
-// 32 of K instead of 8).
+// Every operand element is split into three bf16 pieces and the six products above 2^-24 are
+// taken (fp32_pieces.hpp), with fewer fp32 roundings than the fp32 MFMA's (6 accumulating
+// instructions per 32 of K instead of 8).
 //
 // Operands the split cannot represent are recomputed: an infinity, a NaN or a value that rounds
 // past bf16's largest gives a NaN or infinite sum, operands so small that pieces underflow give
@@ -27,33 +23,10 @@
 // 3.5e-7 (K = 768; 0.8 to 0.9 of it at every size measured, K 128 .. 4096).
 #include <algorithm>
 
+#include "fp32_pieces.hpp"
 #include "gemm_split.hpp"
 
 namespace tl {
-
-// Two fp32 values -> their bf16 roundings, packed.
-__device__ __forceinline__ uint32_t pack_bf2(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
-}
-
-// 8 fp32 values -> three 16-byte chunks of bf16 pieces.
-__device__ __forceinline__ void split8(const float (&x)[8], uint4& p1, uint4& p2, uint4& p3) {
-  uint32_t w1[4], w2[4], w3[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = x[2 * i], b = x[2 * i + 1];
-    w1[i] = pack_bf2(a, b);
-    const float ra = a - __uint_as_float(w1[i] << 16), rb = b - __uint_as_float(w1[i] & 0xffff0000u);
-    w2[i] = pack_bf2(ra, rb);
-    const float sa = ra - __uint_as_float(w2[i] << 16), sb = rb - __uint_as_float(w2[i] & 0xffff0000u);
-    w3[i] = pack_bf2(sa, sb);
-  }
-  p1 = make_uint4(w1[0], w1[1], w1[2], w1[3]);
-  p2 = make_uint4(w2[0], w2[1], w2[2], w2[3]);
-  p3 = make_uint4(w3[0], w3[1], w3[2], w3[3]);
-}
 
 template <typename TO, int BM, int BN, int WGM, int WGN, int NBUF>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p, float* part, int full, int splits) {
@@ -159,13 +132,13 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p
 #pragma unroll
       for (int pl = 0; pl < 3; ++pl)
         a[pl] = *reinterpret_cast<const bf16x8*>(B + pl * PLANE + a_frag + i * 16 * BK);
-      // smallest products first; TN independent sums between two uses of one
-      constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+      // smallest products first; one row of fragments at a time (pairs of rows, for more sums
+      // between two products of one, took 30% longer on 4000 x 2304 x 768)
 #pragma unroll
       for (int t = 0; t < 6; ++t)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[PB[t]][j], a[PA[t]], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kPieceB[t]][j], a[kPieceA[t]], acc[i][j], 0, 0, 0);
     }
   };
 
@@ -199,10 +172,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float v = fabsf(acc[i][j][q]);
-          bad = bad || !(v < __builtin_inff()) || (v > 0.f && v < 0x1p-60f);
-        }
+        for (int q = 0; q < 4; ++q) bad = bad || pieces_doubtful(acc[i][j][q]);
     if (__any(bad)) {  // this wave's block again on the fp32 matrix cores (see above)
       const float* Ar[TM];
       const float* Br[TN];
