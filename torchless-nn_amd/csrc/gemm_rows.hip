@@ -233,37 +233,32 @@ static void launch_rows(int tile, dim3 grid, hipStream_t st, const GemmParams& p
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Modelled time (us, without what all choices share) of `splits` K ranges on one tile.
-static float rows_cost(const RowsTile& t, int64_t M, int64_t N, int64_t nslices, int splits, int elem,
-                       int cus) {
-  const int64_t wgs = ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
-  const float stages = (float)ceil_div(ceil_div(nslices, splits), t.wgk);
-  const float one = elem == 2 ? t.start + stages * t.stage1 : t.start32 + stages * t.stage1_32;
-  const float two = elem == 2 ? t.start + stages * t.stage2 : t.start32 + stages * t.stage2_32;
-  const int64_t slots = (int64_t)t.per_cu * cus, full = wgs / slots, rest = wgs % slots;
-  float us = full * (t.per_cu == 1 ? one : two);
-  if (rest) us += rest <= cus ? one : two;
-  // the partial sums: a second launch, and each written and read once
-  if (splits > 1) us += 1.2f + splits * (float)M * N * 8 / 2e6f;
-  return us;
-}
-
-// The cheapest pair among the first `ntiles` tiles.
+// The cheapest pair among the first `ntiles` tiles by modelled time (us, without what all choices
+// share). Up to 50 pairs are priced on every call, in 32-bit arithmetic: about 1 us of host time.
 static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int elem, int ntiles, int cus) {
   RowsPlan best;
-  const int64_t nslices = K / (128 / elem);
+  const uint32_t nslices = (uint32_t)(K / (128 / elem));
+  const float sums = (float)M * (float)N * (8 / 2e6f);  // partial sums written and read, per split
   for (int i = 0; i < ntiles; ++i) {
     const RowsTile& t = kRowsTiles[i];
     if (t.bm > 32 && t.bm >= 2 * M) continue;  // half padding
-    const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-    if (tiles > (1 << 24)) continue;
-    for (int s = 1; s <= 16; ++s) {
-      // each part keeps at least three slices, and the parts fit two rounds of the chip
-      if (s > 1 && (nslices / s < 3 || tiles * s > 4LL * cus)) break;
-      const float us = rows_cost(t, M, N, nslices, s, elem, cus);
+    const uint64_t tiles64 = (uint64_t)(((uint32_t)M + t.bm - 1) / t.bm) * (((uint32_t)N + t.bn - 1) / t.bn);
+    if (tiles64 > (1 << 24)) continue;
+    const uint32_t tiles = (uint32_t)tiles64, slots = (uint32_t)(t.per_cu * cus);
+    const float start = elem == 2 ? t.start : t.start32;
+    const float stage1 = elem == 2 ? t.stage1 : t.stage1_32, stage2 = elem == 2 ? t.stage2 : t.stage2_32;
+    for (const uint32_t s : {1u, 2u, 3u, 4u, 5u, 6u, 8u, 10u, 12u, 16u}) {
+      // each part keeps at least three slices, and the parts fit four workgroups per CU
+      if (s > 1 && (nslices < 3 * s || tiles * s > 4u * (uint32_t)cus)) break;
+      const float stages = (float)(((nslices + s - 1) / s + t.wgk - 1) / t.wgk);
+      const float one = start + stages * stage1, two = start + stages * stage2;
+      const uint32_t full = tiles * s / slots, rest = tiles * s - full * slots;
+      float us = (float)full * (t.per_cu == 1 ? one : two);
+      if (rest) us += rest <= (uint32_t)cus ? one : two;
+      if (s > 1) us += 2.0f + (float)s * sums;  // and a second launch, on the host as well
       if (best.tile < 0 || us < best.us) {
         best.tile = i;
-        best.splits = s;
+        best.splits = (int)s;
         best.us = us;
       }
     }

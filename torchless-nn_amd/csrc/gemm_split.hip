@@ -251,31 +251,31 @@ static void launch_split(const SplitPlan& plan, dim3 grid, hipStream_t st, const
   else launch_split_tile<TO, 128, 64, 2, 2, 1>(grid, st, p, part, plan);
 }
 
-static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 SplitPlan gemm_split_plan(int64_t M, int64_t N, int64_t K, int cus) {
   SplitPlan best;
-  const int64_t nk = K / 32;
+  const uint32_t nk = (uint32_t)(K / 32);
   for (int i = 0; i < 2; ++i) {
     const SplitTile& t = kSplitTiles[i];
-    const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn), slots = (int64_t)t.per_cu * cus;
-    if (t.bm >= 4 * M || tiles > (1 << 24)) continue;
-    auto round = [&](int64_t wgs, int64_t steps) {  // one round of at most `slots` workgroups
-      return wgs ? t.start + steps * t.step[(wgs - 1) / cus] : 0.f;
+    const uint64_t tiles64 = (uint64_t)(((uint32_t)M + t.bm - 1) / t.bm) * (((uint32_t)N + t.bn - 1) / t.bn);
+    if (t.bm >= 4 * M || tiles64 > (1 << 24)) continue;
+    const uint32_t tiles = (uint32_t)tiles64, slots = (uint32_t)(t.per_cu * cus);
+    auto round = [&](uint32_t wgs, uint32_t steps) {  // one round of at most `slots` workgroups
+      return wgs ? t.start + (float)steps * t.step[(wgs - 1) / (uint32_t)cus] : 0.f;
     };
-    const int64_t rounds = tiles / slots, rest = tiles % slots;
+    const uint32_t rounds = tiles / slots, rest = tiles - rounds * slots;
     // What the whole rounds leave would hold the chip for a round however few tiles it is: its
     // tiles may be split over K, for a reduce launch and their partial sums written and read
     // (4000 x 2304 x 768, 288 tiles of 256x128 on 256 CUs: 112.6 us whole, 83.9 with the last
     // 32 in eight parts each; 2331 x 768 x 3072, 60 tiles: 178 whole, 69.9 in four parts).
-    for (int s : {1, 2, 3, 4, 6, 8}) {
-      if (s > 1 && (rest == 0 || nk / s < 3 || rest * s * 5 > slots * 11)) break;
-      const int64_t per = ceil_div(nk, s), pieces = rest * s;
-      float us = rounds * round(slots, nk) + (pieces / slots) * round(slots, per) + round(pieces % slots, per);
-      if (s > 1) us += 2.4f + (float)(pieces * t.bm * t.bn) * 8 / 4.9e6f;
+    for (const uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+      if (s > 1 && (rest == 0 || nk < 3 * s || rest * s * 5 > slots * 11)) break;
+      const uint32_t per = (nk + s - 1) / s, pieces = rest * s, more = pieces / slots;
+      float us = (float)rounds * round(slots, nk) + (float)more * round(slots, per) +
+                 round(pieces - more * slots, per);
+      if (s > 1) us += 3.0f + (float)(pieces * (uint32_t)(t.bm * t.bn / 1024)) * (8192 / 4.9e6f);
       if (best.tile < 0 || us < best.us) {
         best.tile = i;
-        best.splits = (int)ceil_div(nk, per);
+        best.splits = (int)((nk + per - 1) / per);
         best.full = (int)(best.splits == 1 ? tiles : tiles - rest);
         best.us = us;
       }

@@ -50,11 +50,14 @@ def _packed_nk(w, prenorm=None):
     return packed
 
 
-def _warm(*weights):
-    """Name the weights of the products that follow the next norm launch to that launch
-    (xp.prefetch_hint), so they arrive from the device caches rather than HBM. bf16 weights
-    are read by the products as their packed [N, K] copies, which are the ones named; the
-    other dtypes are left alone."""
+def _warm(rows, *weights):
+    """Name the weights of the products that follow the next norm launch (over `rows` rows) to
+    that launch (xp.prefetch_hint), so they arrive from the device caches rather than HBM. bf16
+    weights are read by the products as their packed [N, K] copies, which are the ones named;
+    the other dtypes are left alone. A norm ignores the list in fewer than 256 workgroups, of at
+    least 4 rows each."""
+    if rows <= 4 * 255:
+        return
     for w in weights:
         if w.dtype is xp.bfloat16:
             xp.prefetch_hint(_packed_nk(w))
@@ -97,10 +100,12 @@ def linear(x2d, w, bias=None, act=xp.TL_ACT_NONE, residual=None, out=None, qkv=N
     Kw, N = w.shape
     if Kw != K:
         raise ValueError(f"matmul shape mismatch: {x2d.shape} @ {w.shape}")
-    fold = prenorm if _folds_gain(prenorm, w.dtype) else None
-    x2d, norm_eps = _prenorm(x2d, prenorm, w.dtype)
+    fold = norm_eps = None
+    if prenorm is not None:
+        fold = prenorm if _folds_gain(prenorm, w.dtype) else None
+        x2d, norm_eps = _prenorm(x2d, prenorm, w.dtype)
     if qkv is None and out is None:
-        out = xp.empty((M, N), x2d.dtype)
+        out = xp.DeviceTensor._alloc((M, N), x2d.dtype, M, N)
     # bf16 always; fp32 when a matrix-core kernel takes the product, which reads B as [N, K]:
     # K % 4 == 0 and either at least 128 output tiles of 128x128 or K <= 1024 with 8 or more
     # 64x64 tiles, or any other K % 32 == 0 (24 x 768 x 3072: 37 us on the vector ALUs, 14 us
@@ -213,20 +218,21 @@ class MultiHeadAttention(Layer):
             raise ValueError(f"sequence length {T} exceeds the context length "
                              f"{self.context_length} of the causal mask")
         dt = input.dtype
-        x2 = input.reshape(B * T, C)
+        x2 = input._rows()
         # the fused kernel takes keys/values with a capacity that is a multiple of 8; the
         # padding positions are never written and never read as values
         fused = self.fused and xp.attention_supported(dt, D, _round_up(T, 8))
         L = _round_up(T, 8) if fused else T
-        q = xp.empty((B, H, T, D), dt)
-        k = xp.empty((B, H, L, D), dt)
-        vt = xp.empty((B, H, D, L), dt)
+        alloc = xp.DeviceTensor._alloc
+        q = alloc((B, H, T, D), dt, B * H * T, D)
+        k = alloc((B, H, L, D), dt, B * H * L, D)
+        vt = alloc((B, H, D, L), dt, B * H * D, L)
         linear(x2, self.qkv_weights, self.qkv_bias, qkv=(q, k, vt, T, H, H, D, L, 0))
         self.query, self.key_t, self.value = q, k, vt
 
         divisor = float(np.float32(D ** 0.5))  # reference layers.py:293 divides by sqrt(D)
         if fused:
-            heads = xp.empty((B, T, C), dt)
+            heads = alloc((B, T, C), dt, B * T, C)
             if self.attn_dropout.dropout_rate > 0.0 and not self.attn_dropout.eval_mode:
                 self.attn_dropout.forward(heads)  # raises: no dropout sampling at inference
             xp.attention(q, k, vt, heads, n_heads_q=H, n_heads_kv=H, divisor=divisor,
@@ -236,9 +242,9 @@ class MultiHeadAttention(Layer):
             heads = self._unfused(q, k, vt, B, T, C, H, D, dt, divisor)
         self.heads_out = heads
 
-        out = linear(heads.reshape(B * T, C), self.out_weights, self.out_bias,
-                     residual=(residual.reshape(B * T, C) if residual is not None else None))
-        self.output = out.reshape(B, T, C)
+        out = linear(heads._rows(), self.out_weights, self.out_bias,
+                     residual=(residual._rows() if residual is not None else None))
+        self.output = out._reshaped((B, T, C), C)
         return self.res_dropout.forward(self.output)
 
     def _forward_cached(self, input, residual, cache, layer, pos0):
@@ -254,12 +260,12 @@ class MultiHeadAttention(Layer):
             self.attn_dropout.forward(input)  # raises: no dropout sampling at inference
         dt, L, Tk = input.dtype, cache.capacity, pos0 + T
         k, vt = cache.k[layer], cache.vt[layer]
-        q = xp.empty((B, H, T, D), dt)
-        linear(input.reshape(B * T, C), self.qkv_weights, self.qkv_bias,
+        q = xp.DeviceTensor._alloc((B, H, T, D), dt, B * H * T, D)
+        linear(input._rows(), self.qkv_weights, self.qkv_bias,
                qkv=(q, k, vt, T, H, H, D, L, pos0))
         self.query, self.key_t, self.value = q, k, vt
         divisor = float(np.float32(D ** 0.5))
-        heads = xp.empty((B, T, C), dt)
+        heads = xp.DeviceTensor._alloc((B, T, C), dt, B * T, C)
         if self.fused and xp.attention_supported(dt, D, L):
             xp.attention(q, k, vt, heads, n_heads_q=H, n_heads_kv=H, divisor=divisor,
                          causal=True, offset=pos0, seq_k=Tk)
@@ -268,9 +274,9 @@ class MultiHeadAttention(Layer):
             self.softmax = _attend_cache_unfused(q, k, vt, heads, B, T, Tk, L, H, H, D, dt,
                                                  divisor, pos0)
         self.heads_out = heads
-        out = linear(heads.reshape(B * T, C), self.out_weights, self.out_bias,
-                     residual=(residual.reshape(B * T, C) if residual is not None else None))
-        self.output = out.reshape(B, T, C)
+        out = linear(heads._rows(), self.out_weights, self.out_bias,
+                     residual=(residual._rows() if residual is not None else None))
+        self.output = out._reshaped((B, T, C), C)
         return self.res_dropout.forward(self.output)
 
     def _unfused(self, q, k, vt, B, T, C, H, D, dt, divisor):
@@ -323,15 +329,15 @@ class TransformerFeedForward(Layer):
         self.input = input
         shape = input.shape
         C = shape[-1]
-        x2 = input.reshape(-1, C)
+        x2 = input._rows()
         if self.act_code is not None:
             h = linear(x2, self.weights1, self.bias1, act=self.act_code)
         else:
             h = self.activation.forward(linear(x2, self.weights1, self.bias1))
         self.hidden_output = h
         y = linear(h, self.weights2, self.bias2,
-                   residual=(residual.reshape(-1, C) if residual is not None else None))
-        self.output = self.dropout.forward(y.reshape(*shape))
+                   residual=(residual._rows() if residual is not None else None))
+        self.output = self.dropout.forward(y._reshaped(shape, C))
         return self.output
 
     def set_eval(self, eval_mode):
@@ -407,15 +413,16 @@ class TransformerBlock(Layer):
         self.input = input
         # each norm launch also pulls the next two products' weights into the device caches
         # (after a forward's 0.8 GB of logits none of them is left there)
-        _warm(self.attn_block.qkv_weights, self.attn_block.out_weights)
+        rows = input.nrows
+        _warm(rows, self.attn_block.qkv_weights, self.attn_block.out_weights)
         if not self.fuse_residual:
             y = input + self.attn_block._forward(self.pre_attn_norm.forward(input), None, cache,
                                                  layer, pos0)
-            _warm(self.ffn.weights1, self.ffn.weights2)
+            _warm(rows, self.ffn.weights1, self.ffn.weights2)
             self.output = y + self.ffn._forward(self.pre_ffn_norm.forward(y), None)
             return self.output
         y = self.attn_block._forward(self.pre_attn_norm.forward(input), input, cache, layer, pos0)
-        _warm(self.ffn.weights1, self.ffn.weights2)
+        _warm(rows, self.ffn.weights1, self.ffn.weights2)
         self.output = self.ffn._forward(self.pre_ffn_norm.forward(y), residual=y)
         return self.output
 

@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import struct
 
 import numpy as np
 
@@ -136,6 +137,12 @@ class _GemmDesc(ctypes.Structure):
     ]
 
 
+# a descriptor as bytes in one call (a quarter of the constructor's time)
+_GEMM_DESC = struct.Struct("@" + "".join(
+    {ctypes.c_int64: "q", ctypes.c_void_p: "P", ctypes.c_int32: "i", ctypes.c_float: "f"}[t]
+    for _, t in _GemmDesc._fields_) + "0q")
+assert _GEMM_DESC.size == ctypes.sizeof(_GemmDesc)
+
 _P, _I32, _I64, _F32, _F64, _SZ = (ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64,
                                    ctypes.c_float, ctypes.c_double, ctypes.c_size_t)
 # name -> argtypes; every function returns int (tl_status) unless listed in _RESTYPES.
@@ -185,7 +192,7 @@ SIGNATURES = {
     "tl_rope2_fwd": [_P, _P, _P, _I64, _I64, _P, _P, _I64, _I64, _P, _I64, _I64, _I32],
     "tl_act_fwd": [_P, _P, _P, _I64, _I32, _I32],
     "tl_argmax": [_P, _P, _I64, _I64, _I64, _I32, _P],
-    "tl_gemm": [_P, ctypes.POINTER(_GemmDesc)],
+    "tl_gemm": [_P, _P],
     "tl_attention_fwd": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                          _F32, _I32, _I64, _I32],
     "tl_attention_fwd_noalloc": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
@@ -256,6 +263,7 @@ class Context:
         self.handle = h
         self.device = device
         self.lib = lib
+        self.malloc, self.free = lib.tl_malloc, lib.tl_free
         self.capturing = False  # between tl_graph_begin and tl_graph_end
 
     def sync(self):
@@ -305,15 +313,17 @@ class DeviceBuffer:
     __slots__ = ("ptr", "nbytes", "_ctx", "version", "__weakref__")
 
     def __init__(self, nbytes: int):
-        c = ctx()
+        c = _ctx or ctx()
         p = ctypes.c_void_p()
-        check(c.lib.tl_malloc(c.handle, int(nbytes), ctypes.byref(p)))
-        self.ptr, self.nbytes, self._ctx, self.version = p.value, int(nbytes), c, 0
+        rc = c.malloc(c.handle, nbytes, ctypes.byref(p))
+        if rc:
+            check(rc)
+        self.ptr, self.nbytes, self._ctx, self.version = p.value, nbytes, c, 0
 
     def __del__(self):
         try:
             if self.ptr:
-                self._ctx.lib.tl_free(self._ctx.handle, self.ptr)
+                self._ctx.free(self._ctx.handle, self.ptr)
                 self.ptr = None
         except Exception:
             pass
@@ -322,14 +332,18 @@ class DeviceBuffer:
 def _prod(shape):
     n = 1
     for s in shape:
-        n *= int(s)
+        n *= s
     return n
 
 
 def _norm_shape(shape):
-    if isinstance(shape, (int, np.integer)):
-        return (int(shape),)
-    return tuple(int(s) for s in shape)
+    """`shape` as a tuple of ints (as it is when it is one)."""
+    if type(shape) is not tuple:
+        shape = (shape,) if isinstance(shape, (int, np.integer)) else tuple(shape)
+    for s in shape:
+        if type(s) is not int:
+            return tuple(int(v) for v in shape)
+    return shape
 
 
 class DeviceTensor:
@@ -337,25 +351,58 @@ class DeviceTensor:
     rows of the last dimension. Rows are padded only where a kernel benefits (e.g. the
     50257-wide logits use a pitch that keeps every row 16-byte aligned)."""
 
-    __slots__ = ("shape", "dtype", "pitch", "buf", "offset", "_aux", "__weakref__")
+    # ptr (buf.ptr + offset), size, nrows and ncols follow from the others and are kept: a
+    # launch reads them several times, and a forward of a small model is all launches
+    __slots__ = ("shape", "dtype", "pitch", "buf", "offset", "ptr", "size", "nrows", "ncols",
+                 "_aux", "__weakref__")
 
     def __init__(self, shape, dtype, pitch=None, buf=None, offset=0):
-        self.shape = _norm_shape(shape)
-        self.dtype = as_dtype(dtype)
-        cols = self.shape[-1] if self.shape else 1
-        self.pitch = int(pitch) if pitch is not None else cols
-        if self.pitch < cols:
+        self.shape = shape = _norm_shape(shape)
+        self.dtype = dtype = dtype if type(dtype) is DType else as_dtype(dtype)
+        self.ncols = cols = shape[-1] if shape else 1
+        self.nrows = rows = _prod(shape[:-1])
+        self.size = rows * cols
+        if pitch is None:
+            pitch = cols
+        elif pitch < cols:
             raise ValueError("pitch smaller than the last dimension")
+        self.pitch = int(pitch)
         if buf is None:
-            buf = DeviceBuffer(max(1, self.nrows * self.pitch * self.dtype.itemsize))
+            buf = DeviceBuffer(int(max(1, rows * pitch * dtype.itemsize)))
         elif self.size:
             # a view must lie inside its buffer: kernels take raw pointers and cannot check
-            end = int(offset) + ((self.nrows - 1) * self.pitch + cols) * self.dtype.itemsize
-            if int(offset) < 0 or end > buf.nbytes:
+            end = offset + ((rows - 1) * pitch + cols) * dtype.itemsize
+            if offset < 0 or end > buf.nbytes:
                 raise ValueError(f"view of {end - int(offset)} bytes at offset {int(offset)} "
                                  f"exceeds its {buf.nbytes}-byte buffer")
         self.buf, self.offset = buf, int(offset)
+        self.ptr = buf.ptr + self.offset
         self._aux = None  # device-side derived data (e.g. a packed weight), by _version
+
+    @staticmethod
+    def _alloc(shape, dtype, nrows, ncols):
+        """A contiguous tensor of `nrows` rows of `ncols`, `shape` (a tuple of ints) known to
+        hold that many."""
+        t = object.__new__(DeviceTensor)
+        t.shape, t.dtype, t.nrows, t.ncols, t.pitch = shape, dtype, nrows, ncols, ncols
+        t.size = n = nrows * ncols
+        t.buf = buf = DeviceBuffer(n * dtype.itemsize or 1)
+        t.offset, t.ptr, t._aux = 0, buf.ptr, None
+        return t
+
+    def _rows(self):
+        """The same rows as a 2-d tensor."""
+        return self._reshaped((self.nrows, self.ncols), self.ncols)
+
+    def _reshaped(self, shape, ncols):
+        """The same elements under a shape of the same size (rows of the same pitch, or a
+        contiguous tensor's)."""
+        t = object.__new__(DeviceTensor)
+        t.shape, t.dtype, t.buf, t.offset, t.ptr = shape, self.dtype, self.buf, self.offset, self.ptr
+        t.size, t.ncols, t._aux = self.size, ncols, None
+        t.nrows = self.nrows if ncols == self.ncols else _prod(shape[:-1])
+        t.pitch = self.pitch if ncols == self.ncols else ncols
+        return t
 
     @property
     def _version(self) -> int:
@@ -369,24 +416,8 @@ class DeviceTensor:
 
     # -- geometry
     @property
-    def ptr(self) -> int:
-        return self.buf.ptr + self.offset
-
-    @property
     def ndim(self):
         return len(self.shape)
-
-    @property
-    def size(self):
-        return _prod(self.shape)
-
-    @property
-    def ncols(self):
-        return self.shape[-1] if self.shape else 1
-
-    @property
-    def nrows(self):
-        return _prod(self.shape[:-1]) if self.shape else 1
 
     @property
     def nbytes(self):
@@ -475,19 +506,17 @@ class DeviceTensor:
     def reshape(self, *shape):
         if len(shape) == 1 and not isinstance(shape[0], (int, np.integer)):
             shape = tuple(shape[0])
-        shape = list(int(s) for s in shape)
+        shape = _norm_shape(shape)
         if -1 in shape:
             i = shape.index(-1)
-            rest = _prod(shape[:i] + shape[i + 1:])
-            shape[i] = self.size // rest if rest else 0
-        shape = tuple(shape)
+            rest = _prod(shape[:i]) * _prod(shape[i + 1:])
+            shape = shape[:i] + (self.size // rest if rest else 0,) + shape[i + 1:]
         if _prod(shape) != self.size:
             raise ValueError(f"cannot reshape {self.shape} into {shape}")
-        if shape and self.shape and shape[-1] == self.ncols:
-            return DeviceTensor(shape, self.dtype, self.pitch, self.buf, self.offset)
-        if not self.contiguous:
+        ncols = shape[-1] if shape else 1
+        if not (shape and self.shape and ncols == self.ncols) and not self.contiguous:
             raise ValueError("reshape of a padded tensor must keep the last dimension")
-        return DeviceTensor(shape, self.dtype, None, self.buf, self.offset)
+        return self._reshaped(shape, ncols)
 
     def fill(self, value):
         if not self.contiguous:
@@ -724,7 +753,7 @@ class random:  # noqa: N801  (mirrors `xp.random`)
 
 # ---- kernel wrappers used by the layers ------------------------------------------------
 def _c():
-    c = ctx()
+    c = _ctx or ctx()
     return c.lib, c.handle
 
 
@@ -737,7 +766,7 @@ def gemm(A: DeviceTensor, B: DeviceTensor, *, M, N, K, lda, ldb, b_layout, C=Non
     read on the device when the kernel runs). norm_eps (M <= 16) scales each row of the
     product by 1 / sqrt(mean(A_row^2) + norm_eps): RMSNorm(A) @ B when B carries the norm's
     gain."""
-    pos_dev = None
+    pos_dev = 0
     if qkv is not None:
         q, k, vt, T, Hq, Hkv, Dh = qkv[:7]
         kv_len, kv_pos0 = (qkv[7], qkv[8]) if len(qkv) > 7 else (0, 0)
@@ -746,33 +775,38 @@ def gemm(A: DeviceTensor, B: DeviceTensor, *, M, N, K, lda, ldb, b_layout, C=Non
         epi, qp, kp, vp = TL_EPI_QKV_SPLIT, q.ptr, k.ptr, vt.ptr
     else:
         epi = TL_EPI_GEGLU if geglu else TL_EPI_STORE
-        qp = kp = vp = None
+        qp = kp = vp = 0
         T = Hq = Hkv = Dh = kv_len = kv_pos0 = 0
     code_in = A.dtype.code
-    # one positional constructor call, in the field order of _GemmDesc
-    d = _GemmDesc(M, N, K, A.ptr, lda, B.ptr, ldb, b_layout,
-                  C.ptr if C is not None else None, ldc, code_in,
-                  as_dtype(out_dtype).code if out_dtype is not None else code_in,
-                  batch, batch_inner, sa[0], sa[1], sb[0], sb[1], sc[0], sc[1],
-                  bias.ptr if bias is not None else None,
-                  residual.ptr if residual is not None else None, ldr, sr[0], sr[1],
-                  act, float(divisor), epi, qp, kp, vp, T, Hq, Hkv, Dh, kv_len, kv_pos0,
-                  KFAMILY[family], GEMM_TILES[tile], pos_dev, int(norm_eps is not None),
-                  float(norm_eps) if norm_eps is not None else 0.0)
+    # in the field order of _GemmDesc
+    d = _GEMM_DESC.pack(M, N, K, A.ptr, lda, B.ptr, ldb, b_layout,
+                        C.ptr if C is not None else 0, ldc, code_in,
+                        as_dtype(out_dtype).code if out_dtype is not None else code_in,
+                        batch, batch_inner, sa[0], sa[1], sb[0], sb[1], sc[0], sc[1],
+                        bias.ptr if bias is not None else 0,
+                        residual.ptr if residual is not None else 0, ldr, sr[0], sr[1],
+                        act, divisor, epi, qp, kp, vp, T, Hq, Hkv, Dh, kv_len, kv_pos0,
+                        KFAMILY[family], GEMM_TILES[tile], pos_dev, norm_eps is not None,
+                        norm_eps if norm_eps is not None else 0.0)
     lib_, h = _c()
-    check(lib_.tl_gemm(h, ctypes.byref(d)))
+    rc = lib_.tl_gemm(h, d)
+    if rc:
+        check(rc)
     if qkv is not None:
         _wrote(qkv[0], qkv[1], qkv[2])
-    else:
-        _wrote(C)
+    elif C is not None:
+        C.buf.version += 1
 
 
 def layernorm(x: DeviceTensor, gamma, beta, eps, out=None):
-    out = out if out is not None else DeviceTensor(x.shape, x.dtype)
+    if out is None:
+        out = DeviceTensor._alloc(x.shape, x.dtype, x.nrows, x.ncols)
     lib_, h = _c()
-    check(lib_.tl_layernorm_fwd(h, x.ptr, gamma.ptr, beta.ptr, out.ptr, x.nrows, x.ncols,
-                                x.pitch, out.pitch, float(eps), x.dtype.code))
-    _wrote(out)
+    rc = lib_.tl_layernorm_fwd(h, x.ptr, gamma.ptr, beta.ptr, out.ptr, x.nrows, x.ncols,
+                               x.pitch, out.pitch, eps, x.dtype.code)
+    if rc:
+        check(rc)
+    out.buf.version += 1
     return out
 
 
@@ -949,10 +983,12 @@ def attention(q: DeviceTensor, k: DeviceTensor, vt: DeviceTensor, out: DeviceTen
     Lk = k.shape[2]
     Tk = Lk if seq_k is None else seq_k
     lib_, h = _c()
-    check(lib_.tl_attention_fwd(h, q.ptr, k.ptr, vt.ptr, out.ptr, B, n_heads_q, n_heads_kv, Tq,
-                                Tk, D, out.pitch, int(offset), float(divisor), int(bool(causal)),
-                                Lk, q.dtype.code))
-    _wrote(out)
+    rc = lib_.tl_attention_fwd(h, q.ptr, k.ptr, vt.ptr, out.ptr, B, n_heads_q, n_heads_kv, Tq,
+                               Tk, D, out.pitch, int(offset), divisor, 1 if causal else 0,
+                               Lk, q.dtype.code)
+    if rc:
+        check(rc)
+    out.buf.version += 1
     return out
 
 
