@@ -258,3 +258,51 @@ def test_fp32_attention_pieces_not_finite(xp, D):
         assert ref.max_rel(got[..., cols], want[..., cols]) <= 4e-6, cols
     assert ref.max_rel(got[0, :144, 3], want[0, :144, 3]) <= 4e-6
     assert ref.max_rel(got[0, :176, 4], want[0, :176, 4]) <= 4e-6
+
+
+# 256x256 tiles that fill the chip: one to many K steps (odd and even counts), remainders of rows
+# and columns, more than one round, a K beyond the late-load form's
+@pytest.mark.parametrize("mnk", [(8192, 2048, 256), (8192, 2048, 320), (4096, 4096, 384),
+                                 (7950, 2000, 2048), (2048, 8192, 8256), (16384, 4104, 256)])
+def test_half_tiles_in_turn(xp, mnk):
+    M, N, K = mnk
+    a, w, bias, res = inputs(xp, "bf16", M, N, K)
+    da, dw, db, dres = (xp.array(t, dtype="bf16") for t in (a, w, bias, res))
+    rows = np.unique(np.r_[0:3, 120:132, 250:260, M - 140:M - 120, M - 3:M])
+    y = a[rows].astype(np.float64) @ w.astype(np.float64).T
+    for kind in ("plain", "silu", "residual"):
+        out = xp.empty((M, N), "bf16")
+        kw, want = {}, y
+        if kind != "plain":
+            kw, want = dict(bias=db), y + bias
+        if kind == "silu":
+            kw["act"], want = xp.TL_ACT_SILU, ref.silu(want).astype(np.float64)
+        if kind == "residual":
+            kw.update(residual=dres, ldr=N)
+            want = want + res[rows]
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=out, ldc=N, **kw)
+        old = xp.empty((M, N), "bf16")  # a named tile: the same sums in the same order
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=old, ldc=N,
+                tile="dma128x128", **kw)
+        assert np.array_equal(out.get_raw(), old.get_raw()), (mnk, kind)
+        assert ref.max_rel(out.get()[rows], want) <= bar("bf16", K), (mnk, kind)
+
+
+def test_half_tiles_in_turn_scatter_and_gated(xp):
+    """The QKV scatter (slabs inside one part and across parts) and the gated epilogue on the
+    same tiles, bit for bit against a named tile."""
+    B, T, Hq, Hkv, D, K = 32, 256, 12, 2, 128, 256
+    M, N = B * T, (Hq + 2 * Hkv) * D
+    a, w, bias, _ = inputs(xp, "bf16", M, N, K)
+    da, dw, db = (xp.array(t, dtype="bf16") for t in (a, w, bias))
+    got = []
+    for tile in ("auto", "dma128x128"):
+        q, k, vt = (xp.empty(s, "bf16").fill(3) for s in ((B, Hq, T, D), (B, Hkv, T, D), (B, Hkv, D, T)))
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, bias=db, tile=tile,
+                qkv=(q, k, vt, T, Hq, Hkv, D, T, 0))
+        out = xp.empty((M, N // 2), "bf16")
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK, C=out, ldc=N // 2, tile=tile,
+                act=xp.TL_ACT_GELU, geglu=True)
+        got.append([t.get_raw() for t in (q, k, vt, out)])
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
