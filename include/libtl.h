@@ -86,7 +86,7 @@ enum tl_gemm_tile {
   TL_TILE_PERSIST_256x128_W8 = 12,
   TL_TILE_PERSIST_128x128 = 13,
   /* weight streaming for M <= 16 (decode steps): 16 rows of B per workgroup, K split over
-   * its 8 waves; chosen by TL_TILE_AUTO whenever M <= 16 */
+   * its waves; chosen by TL_TILE_AUTO for M <= 16 up to 32767 columns */
   TL_TILE_SKINNY = 14,
   TL_TILE_DMA_256x256_W8 = 15, /* direct global->LDS, 8 waves of 128x64, 2 stages */
   TL_TILE_DMA_128x96 = 16,     /* direct global->LDS, 4 waves of 64x48, 2 stages */

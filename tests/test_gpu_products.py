@@ -306,3 +306,32 @@ def test_half_tiles_in_turn_scatter_and_gated(xp):
         got.append([t.get_raw() for t in (q, k, vt, out)])
     for x, y in zip(*got):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("D,Hkv", [(256, 1), (128, 2), (64, 4)])
+@pytest.mark.parametrize("pos", [0, 63, 64, 500, 1023])
+def test_decode_trims_dead_blocks(xp, D, Hkv, pos):
+    """A grid of more than one round at a device position: only live key blocks are read (the
+    others hold NaN), several per workgroup, also when the position reaches the capacity; the
+    rotated new key is written back."""
+    B, L, Hq = 160, 1024, 8
+    rng = np.random.default_rng(pos + D)
+    r = ref.round_bf16
+    q = r(rng.standard_normal((B, Hq, 1, D), dtype=F32))
+    k, vt = (r(rng.standard_normal(s, dtype=F32)) for s in ((B, Hkv, L, D), (B, Hkv, D, L)))
+    k[:, :, pos + 1:], vt[..., pos + 1:] = np.nan, np.nan
+    dk = xp.array(k, dtype="bf16")
+    out = xp.empty((B, 1, Hq * D), "bf16")
+    xp.attention_decode_dev(xp.array(q, dtype="bf16"), dk, xp.array(vt, dtype="bf16"), out,
+                            xp.array(np.array([pos], np.int64)), n_heads_q=Hq, n_heads_kv=Hkv,
+                            divisor=float(F32(D ** 0.5)), rope=xp.rope_table(1, D, 10000.0, pos))
+    cos, sin = ref.rope_table(1, D, 10000.0, pos)
+    qr = r(ref.rope(q, cos, sin))
+    k[:, :, pos:pos + 1] = r(ref.rope(k[:, :, pos:pos + 1], cos, sin))
+    some = [0, 1, 77, B - 1]
+    want = attention_exact(qr[some], k[some], vt[some], True, pos, pos + 1)
+    assert ref.max_rel(out.get()[some], want) <= 2e-2
+    assert np.isfinite(out.get()).all()
+    got = dk.get()
+    assert np.array_equal(np.isnan(got), np.isnan(k))
+    assert ref.max_rel(np.nan_to_num(got), np.nan_to_num(k)) <= 2.0 ** -7

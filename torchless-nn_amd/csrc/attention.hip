@@ -590,18 +590,25 @@ __device__ __forceinline__ uint2 keep_below(uint2 v, int n) {
 struct DecodeWs {
   float* o;   // [B*Hkv][nblk][16][D] unnormalised partial outputs
   float* ml;  // [B*Hkv][nblk][16][2] (max in log2 units, sum)
-  int nblk;
+  int nblk, keys;  // blocks of keys, keys per block
+  int trim;        // with a device position: blocks past the live keys are left out
 };
 
-template <int D, int NW, int J>
+template <int D, int NW, int J, bool TRIM>
 __global__ __launch_bounds__(64 * NW) void attention_decode_kernel(AttnParams p, DecodeWs w) {
   static_assert(J == 2 || J == 4, "16-key tiles per wave: 2 or 4");
-  if (p.pos_dev) {  // the grid covers the capacity; blocks past the live keys write empty partials
+  constexpr int KS = D / 32, DT = D / 16, KPW = 16 * J;
+  if (p.pos_dev) {
     const int64_t pos = *p.pos_dev;
     p.offset = pos;
     p.Tk = (int)min(pos + (int64_t)p.Tq, (int64_t)p.Lk);
   }
-  constexpr int KS = D / 32, DT = D / 16, KPW = 16 * J;
+  // With TRIM (a device position and a grid of more than one round: large batches, long caches)
+  // this workgroup takes key blocks blockIdx.x, + gridDim.x, ... up to the live keys, at the price
+  // of waiting for the position before the first load; otherwise block blockIdx.x, and blocks past
+  // the live keys write empty partials.
+  const int live = (p.Tk + NW * KPW - 1) / (NW * KPW);
+  if (TRIM && (int)blockIdx.x >= live) return;
   __shared__ float sm[NW][16], sl[NW][16];
   __shared__ f32x4 so[NW][DT][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -645,193 +652,202 @@ __global__ __launch_bounds__(64 * NW) void attention_decode_kernel(AttnParams p,
   }
   const bf16_t* kh = p.k + (int64_t)bh * p.Lk * D;
   const bf16_t* vh = p.vt + (int64_t)bh * D * p.Lk;
-  const int kc0 = (blockIdx.x * NW + wave) * KPW;
+  int blk = blockIdx.x;
+  do {
+    const bool first = !TRIM || blk == (int)blockIdx.x;
+    const int kc0 = (blk * NW + wave) * KPW;
 
-  // All of this wave's K and V^T fragments are requested up front (the V^T reads do not
-  // depend on the softmax), so the wave waits for one memory round trip, not two. The
-  // addresses are clamped to the cache capacity and do not depend on the live key count, so
-  // with a device position the loads do not wait for it either; keys at or past Tk (cache
-  // rows never written: any bits, NaN included) are masked out of the scores by a select and
-  // their values zeroed below. A wave whose keys all lie past Tk reads a few such rows.
-  bf16x8 kf[J][KS];
-  // V^T rows in the key order of the P.V B operand: keys 32 hp + 4 grp + 0..3 and
-  // 32 hp + 16 + 4 grp + 0..3 (values past Tk zeroed, since 0 * NaN would not be 0; the
-  // capacity is a multiple of 8, so a 4-key run that starts inside it ends inside it)
-  uint2 vfa[J / 2][DT], vfb[J / 2][DT];
+    // All of this wave's K and V^T fragments are requested up front (the V^T reads do not
+    // depend on the softmax), so the wave waits for one memory round trip, not two. The
+    // addresses are clamped to the cache capacity and do not depend on the live key count, so
+    // with a device position (and no trim) the loads do not wait for it either; keys at or past Tk (cache
+    // rows never written: any bits, NaN included) are masked out of the scores by a select and
+    // their values zeroed below. A wave whose keys all lie past Tk reads a few such rows.
+    bf16x8 kf[J][KS];
+    // V^T rows in the key order of the P.V B operand: keys 32 hp + 4 grp + 0..3 and
+    // 32 hp + 16 + 4 grp + 0..3 (values past Tk zeroed, since 0 * NaN would not be 0; the
+    // capacity is a multiple of 8, so a 4-key run that starts inside it ends inside it)
+    uint2 vfa[J / 2][DT], vfb[J / 2][DT];
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int key = min(kc0 + 16 * j + col, p.Lk - 1);
-    const bf16_t* krow = kh + (int64_t)key * D + 8 * grp;
+    for (int j = 0; j < J; ++j) {
+      const int key = min(kc0 + 16 * j + col, p.Lk - 1);
+      const bf16_t* krow = kh + (int64_t)key * D + 8 * grp;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kf[j][ks] = *reinterpret_cast<const bf16x8*>(krow + 32 * ks);
-  }
-#pragma unroll
-  for (int hp = 0; hp < J / 2; ++hp) {
-    const int ka = min(kc0 + 32 * hp + 4 * grp, p.Lk - 4), kb = min(kc0 + 32 * hp + 16 + 4 * grp, p.Lk - 4);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const bf16_t* vrow = vh + (int64_t)(dt * 16 + col) * p.Lk;
-      vfa[hp][dt] = *reinterpret_cast<const uint2*>(vrow + ka);
-      vfb[hp][dt] = *reinterpret_cast<const uint2*>(vrow + kb);
+      for (int ks = 0; ks < KS; ++ks) kf[j][ks] = *reinterpret_cast<const bf16x8*>(krow + 32 * ks);
     }
-  }
-  if (!rowok) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = zero;
-  }
-  if constexpr (KH > 0) {
-    if (p.rope) {
+    for (int hp = 0; hp < J / 2; ++hp) {
+      const int ka = min(kc0 + 32 * hp + 4 * grp, p.Lk - 4), kb = min(kc0 + 32 * hp + 16 + 4 * grp, p.Lk - 4);
 #pragma unroll
-      for (int ks = 0; ks < KH; ++ks) rope8v(qf[ks], qf[ks + KH], qcs[ks]);
+      for (int dt = 0; dt < DT; ++dt) {
+        const bf16_t* vrow = vh + (int64_t)(dt * 16 + col) * p.Lk;
+        vfa[hp][dt] = *reinterpret_cast<const uint2*>(vrow + ka);
+        vfb[hp][dt] = *reinterpret_cast<const uint2*>(vrow + kb);
+      }
     }
-  }
-  // zero the values of keys >= Tk (unrotated key index: keys 32 hp + 4 grp + i)
+    if (first) {
+      if (!rowok) {
 #pragma unroll
-  for (int hp = 0; hp < J / 2; ++hp) {
-    const int na = p.Tk - (kc0 + 32 * hp + 4 * grp), nb = na - 16;
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = zero;
+      }
+      if constexpr (KH > 0) {
+        if (p.rope) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      vfa[hp][dt] = keep_below(vfa[hp][dt], na);
-      vfb[hp][dt] = keep_below(vfb[hp][dt], nb);
+          for (int ks = 0; ks < KH; ++ks) rope8v(qf[ks], qf[ks + KH], qcs[ks]);
+        }
+      }
+    } else {
+      __syncthreads();  // the merge space of the block before has been read
     }
-  }
-  // fused RoPE of this call's new keys (positions offset .. offset + Tq - 1): the one lane
-  // group holding such a key rotates it and writes it back to the cache for later steps
-  if constexpr (KH > 0) {
-    if (p.rope) {
+    // zero the values of keys >= Tk (unrotated key index: keys 32 hp + 4 grp + i)
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int key = kc0 + 16 * j + col;
-        const int64_t tn = (int64_t)key - p.offset;
-        if (key < p.Tk && tn >= 0 && tn < p.Tq) {
-          const float* cs = p.rope + tn * (D / 2) + 8 * grp;
-          const float* sn = cs + (int64_t)p.Tq * (D / 2);
-          bf16_t* krow = const_cast<bf16_t*>(kh) + (int64_t)key * D + 8 * grp;
-          // the whole table row first, then the rotations and stores (a load after a store
-          // to the cache would wait for it); with one query position (a decode step) the new
-          // key's row is table row 0, which every lane already holds for its query (qcs)
-          float4 kcs[KH][4];
-          if (p.Tq == 1) {
+    for (int hp = 0; hp < J / 2; ++hp) {
+      const int na = p.Tk - (kc0 + 32 * hp + 4 * grp), nb = na - 16;
 #pragma unroll
-            for (int ks = 0; ks < KH; ++ks)
+      for (int dt = 0; dt < DT; ++dt) {
+        vfa[hp][dt] = keep_below(vfa[hp][dt], na);
+        vfb[hp][dt] = keep_below(vfb[hp][dt], nb);
+      }
+    }
+    // fused RoPE of this call's new keys (positions offset .. offset + Tq - 1): the one lane
+    // group holding such a key rotates it and writes it back to the cache for later steps
+    if constexpr (KH > 0) {
+      if (p.rope) {
 #pragma unroll
-              for (int c = 0; c < 4; ++c) kcs[ks][c] = qcs[ks][c];
-          } else {
+        for (int j = 0; j < J; ++j) {
+          const int key = kc0 + 16 * j + col;
+          const int64_t tn = (int64_t)key - p.offset;
+          if (key < p.Tk && tn >= 0 && tn < p.Tq) {
+            const float* cs = p.rope + tn * (D / 2) + 8 * grp;
+            const float* sn = cs + (int64_t)p.Tq * (D / 2);
+            bf16_t* krow = const_cast<bf16_t*>(kh) + (int64_t)key * D + 8 * grp;
+            // the whole table row first, then the rotations and stores (a load after a store
+            // to the cache would wait for it); with one query position (a decode step) the new
+            // key's row is table row 0, which every lane already holds for its query (qcs)
+            float4 kcs[KH][4];
+            if (p.Tq == 1) {
+#pragma unroll
+              for (int ks = 0; ks < KH; ++ks)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) kcs[ks][c] = qcs[ks][c];
+            } else {
+#pragma unroll
+              for (int ks = 0; ks < KH; ++ks) {
+                kcs[ks][0] = *reinterpret_cast<const float4*>(cs + 32 * ks);
+                kcs[ks][1] = *reinterpret_cast<const float4*>(cs + 32 * ks + 4);
+                kcs[ks][2] = *reinterpret_cast<const float4*>(sn + 32 * ks);
+                kcs[ks][3] = *reinterpret_cast<const float4*>(sn + 32 * ks + 4);
+              }
+            }
 #pragma unroll
             for (int ks = 0; ks < KH; ++ks) {
-              kcs[ks][0] = *reinterpret_cast<const float4*>(cs + 32 * ks);
-              kcs[ks][1] = *reinterpret_cast<const float4*>(cs + 32 * ks + 4);
-              kcs[ks][2] = *reinterpret_cast<const float4*>(sn + 32 * ks);
-              kcs[ks][3] = *reinterpret_cast<const float4*>(sn + 32 * ks + 4);
+              rope8v(kf[j][ks], kf[j][ks + KH], kcs[ks]);
+              *reinterpret_cast<bf16x8*>(krow + 32 * ks) = kf[j][ks];
+              *reinterpret_cast<bf16x8*>(krow + 32 * (ks + KH)) = kf[j][ks + KH];
             }
-          }
-#pragma unroll
-          for (int ks = 0; ks < KH; ++ks) {
-            rope8v(kf[j][ks], kf[j][ks + KH], kcs[ks]);
-            *reinterpret_cast<bf16x8*>(krow + 32 * ks) = kf[j][ks];
-            *reinterpret_cast<bf16x8*>(krow + 32 * (ks + KH)) = kf[j][ks + KH];
           }
         }
       }
     }
-  }
 
-  // S^T = K Q^T for J tiles of 16 keys: lane holds keys kc0 + 16 j + 4 grp + i of row col
-  f32x4 s[J];
+    // S^T = K Q^T for J tiles of 16 keys: lane holds keys kc0 + 16 j + 4 grp + i of row col
+    f32x4 s[J];
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < J; ++j) {
+      s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[j][ks], qf[ks], s[j], 0, 0, 0);
-  }
-  float mx = -INFINITY;
-#pragma unroll
-  for (int j = 0; j < J; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = kc0 + 16 * j + 4 * grp + i;
-      const bool ok = rowok && key < p.Tk && (!p.causal || (int64_t)key <= qpos);
-      const float x = ok ? s[j][i] * p.scale_log2 : -INFINITY;
-      s[j][i] = x;
-      mx = fmaxf(mx, x);
+      for (int ks = 0; ks < KS; ++ks)
+        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[j][ks], qf[ks], s[j], 0, 0, 0);
     }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  float sum = 0.f;
+    float mx = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < J; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float e = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[j][i] - mx);
-      s[j][i] = e;
-      sum += e;
-    }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
+      for (int i = 0; i < 4; ++i) {
+        const int key = kc0 + 16 * j + 4 * grp + i;
+        const bool ok = rowok && key < p.Tk && (!p.causal || (int64_t)key <= qpos);
+        const float x = ok ? s[j][i] * p.scale_log2 : -INFINITY;
+        s[j][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[j][i] - mx);
+        s[j][i] = e;
+        sum += e;
+      }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
 
-  // O^T = V^T P^T: B operand = this lane's 8 probabilities (keys 32 hp + 4 grp + 0..3 and
-  // 32 hp + 16 + 4 grp + 0..3), A operand = V^T rows read with the same key order
-  f32x4 o[DT];
+    // O^T = V^T P^T: B operand = this lane's 8 probabilities (keys 32 hp + 4 grp + 0..3 and
+    // 32 hp + 16 + 4 grp + 0..3), A operand = V^T rows read with the same key order
+    f32x4 o[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int hp = 0; hp < J / 2; ++hp) {
-    bf16x8 pf;
+    for (int hp = 0; hp < J / 2; ++hp) {
+      bf16x8 pf;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pf[i] = (__bf16)s[2 * hp][i];
-      pf[4 + i] = (__bf16)s[2 * hp + 1][i];
+      for (int i = 0; i < 4; ++i) {
+        pf[i] = (__bf16)s[2 * hp][i];
+        pf[4 + i] = (__bf16)s[2 * hp + 1][i];
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const uint2 va = vfa[hp][dt], vb = vfb[hp][dt];
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, make_uint4(va.x, va.y, vb.x, vb.y));
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[dt], 0, 0, 0);
+      }
     }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const uint2 va = vfa[hp][dt], vb = vfb[hp][dt];
-      const bf16x8 vf = __builtin_bit_cast(bf16x8, make_uint4(va.x, va.y, vb.x, vb.y));
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[dt], 0, 0, 0);
-    }
-  }
 
-  // merge the 4 waves: rows col, head-dim 16 dt + 4 grp + i
-  if (grp == 0) {
-    sm[wave][col] = mx;
-    sl[wave][col] = sum;
-  }
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) so[wave][dt][lane] = o[dt];
-  __syncthreads();
-  const int64_t slot = (int64_t)bh * w.nblk + blockIdx.x;
-  for (int e = threadIdx.x; e < DT * 64; e += 64 * NW) {
-    const int dt = e >> 6, ln = e & 63, r = ln & 15;
-    if (r >= R) continue;
-    float m = -INFINITY;
-#pragma unroll
-    for (int v = 0; v < NW; ++v) m = fmaxf(m, sm[v][r]);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int v = 0; v < NW; ++v) {
-      const float f = sm[v][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sm[v][r] - m);
-      acc += so[v][dt][ln] * f;
+    // merge the 4 waves: rows col, head-dim 16 dt + 4 grp + i
+    if (grp == 0) {
+      sm[wave][col] = mx;
+      sl[wave][col] = sum;
     }
-    *reinterpret_cast<f32x4*>(w.o + (slot * 16 + r) * D + dt * 16 + 4 * (ln >> 4)) = acc;
-  }
-  if (threadIdx.x < 16) {
-    const int r = threadIdx.x;
-    float m = -INFINITY, l = 0.f;
 #pragma unroll
-    for (int v = 0; v < NW; ++v) m = fmaxf(m, sm[v][r]);
+    for (int dt = 0; dt < DT; ++dt) so[wave][dt][lane] = o[dt];
+    __syncthreads();
+    const int64_t slot = (int64_t)bh * w.nblk + blk;
+    for (int e = threadIdx.x; e < DT * 64; e += 64 * NW) {
+      const int dt = e >> 6, ln = e & 63, r = ln & 15;
+      if (r >= R) continue;
+      float m = -INFINITY;
 #pragma unroll
-    for (int v = 0; v < NW; ++v)
-      l += sm[v][r] == -INFINITY ? 0.f : sl[v][r] * __builtin_amdgcn_exp2f(sm[v][r] - m);
-    w.ml[(slot * 16 + r) * 2] = m;
-    w.ml[(slot * 16 + r) * 2 + 1] = l;
-  }
+      for (int v = 0; v < NW; ++v) m = fmaxf(m, sm[v][r]);
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        const float f = sm[v][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sm[v][r] - m);
+        acc += so[v][dt][ln] * f;
+      }
+      *reinterpret_cast<f32x4*>(w.o + (slot * 16 + r) * D + dt * 16 + 4 * (ln >> 4)) = acc;
+    }
+    if (threadIdx.x < 16) {
+      const int r = threadIdx.x;
+      float m = -INFINITY, l = 0.f;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) m = fmaxf(m, sm[v][r]);
+#pragma unroll
+      for (int v = 0; v < NW; ++v)
+        l += sm[v][r] == -INFINITY ? 0.f : sl[v][r] * __builtin_amdgcn_exp2f(sm[v][r] - m);
+      w.ml[(slot * 16 + r) * 2] = m;
+      w.ml[(slot * 16 + r) * 2 + 1] = l;
+    }
+    blk += gridDim.x;
+  } while (TRIM && blk < live);
 }
 
 // One workgroup per (query row, batch x kv head). Thread d requests its first PF partial
 // outputs of head-dim d and the (max, sum) pair of partial d before anything else (none of
 // these loads depends on another), so the kernel waits for one memory round trip; the
 // maxima give the weights exp2(m_k - max), and the partials are summed with those weights.
-template <int D>
+template <int D, bool TRIM>
 __global__ __launch_bounds__(D < 64 ? 64 : D) void attention_combine_kernel(AttnParams p, DecodeWs w) {
   constexpr int NT = D < 64 ? 64 : D;  // whole waves, so the shuffles see only live lanes
   constexpr int NWV = NT / 64;
@@ -843,8 +859,10 @@ __global__ __launch_bounds__(D < 64 ? 64 : D) void attention_combine_kernel(Attn
   const int b = bh / p.Hkv, hk = bh - b * p.Hkv;
   const int g = p.Hq / p.Hkv;
   const int jh = r / p.Tq, t = r - jh * p.Tq;
-  const int nblk = w.nblk;
-  const int64_t base = (int64_t)bh * nblk;
+  // partials of the live keys (with a device position the later blocks wrote none)
+  int nblk = w.nblk;
+  if constexpr (TRIM) nblk = min(nblk, (int)((min(*p.pos_dev + (int64_t)p.Tq, (int64_t)p.Lk) + w.keys - 1) / w.keys));
+  const int64_t base = (int64_t)bh * w.nblk;
   const float* src = w.o + (base * 16 + r) * D + min(d, D - 1);
   float pre[PF];
 #pragma unroll
@@ -1646,8 +1664,13 @@ constexpr int kDecodeWaves = 2, kDecodeTiles = 2;
 template <int D>
 static void launch_decode(dim3 g1, dim3 g2, hipStream_t st, const AttnParams& p,
                           const DecodeWs& w) {
-  attention_decode_kernel<D, kDecodeWaves, kDecodeTiles><<<g1, 64 * kDecodeWaves, 0, st>>>(p, w);
-  attention_combine_kernel<D><<<g2, D < 64 ? 64 : D, 0, st>>>(p, w);
+  if (w.trim) {
+    attention_decode_kernel<D, kDecodeWaves, kDecodeTiles, true><<<g1, 64 * kDecodeWaves, 0, st>>>(p, w);
+    attention_combine_kernel<D, true><<<g2, D < 64 ? 64 : D, 0, st>>>(p, w);
+  } else {
+    attention_decode_kernel<D, kDecodeWaves, kDecodeTiles, false><<<g1, 64 * kDecodeWaves, 0, st>>>(p, w);
+    attention_combine_kernel<D, false><<<g2, D < 64 ? 64 : D, 0, st>>>(p, w);
+  }
 }
 
 }  // namespace tl
@@ -1743,7 +1766,8 @@ static int attention_fwd(tl_ctx* ctx, const void* q, const void* k, const void* 
     constexpr int nw = kDecodeWaves, jt = kDecodeTiles;
     // with a device position the key count is known only on the device: cover the capacity
     const int64_t keys = pos_dev ? cap : seq_k;
-    w.nblk = (int)((keys + 16 * nw * jt - 1) / (16 * nw * jt));
+    w.keys = 16 * nw * jt;
+    w.nblk = (int)((keys + w.keys - 1) / w.keys);
     TL_REQUIRE(w.nblk <= 1024, "decode attention takes up to %d keys with this split",
                1024 * 16 * nw * jt);
     const int64_t slots = batch * n_heads_kv * w.nblk;
@@ -1775,7 +1799,18 @@ static int attention_fwd(tl_ctx* ctx, const void* q, const void* k, const void* 
     }
     w.o = (float*)ws;
     w.ml = (float*)((char*)ws + obytes);
-    const dim3 g1((unsigned)w.nblk, (unsigned)(batch * n_heads_kv));
+    // With a device position the blocks cover the capacity, live or not. Beyond 8 two-wave
+    // workgroups per CU the live blocks are shared out over 4 per CU (us, 96 x 300 of 4096 keys,
+    // head dim 256: 118 -> 20; 96 x 3000 of 4096: 119 -> 98; 90 x 2 x 200 of 4096, head dim 128:
+    // 111 -> 17; at 6 per CU with most keys live, 48 x 1500 of 2048, 40.4 against 39.9, 24 x 2 x
+    // 1500 of 2048 23.1 against 22.7). With a host position every block is live, and one
+    // workgroup each is the faster form (24 x 12 x 902 keys, head dim 64: 23.5 against 25.3).
+    const int64_t per_round = 4LL * (ctx->num_cus > 0 ? ctx->num_cus : 256);
+    w.trim = pos_dev && batch * n_heads_kv * w.nblk > 2 * per_round;
+    const int64_t per_bh = w.trim ? std::max<int64_t>(1, std::min<int64_t>(w.nblk, (per_round + batch * n_heads_kv - 1) /
+                                                                                       (batch * n_heads_kv)))
+                                  : w.nblk;
+    const dim3 g1((unsigned)per_bh, (unsigned)(batch * n_heads_kv));
     const dim3 g2((unsigned)rows_per_kv, (unsigned)(batch * n_heads_kv));
     switch (head_dim) {
       case 32: launch_decode<32>(g1, g2, ctx->stream, p, w); break;
