@@ -328,10 +328,8 @@ def test_decode_trims_dead_blocks(xp, D, Hkv, pos):
     cos, sin = ref.rope_table(1, D, 10000.0, pos)
     qr = r(ref.rope(q, cos, sin))
     k[:, :, pos:pos + 1] = r(ref.rope(k[:, :, pos:pos + 1], cos, sin))
-    some = [0, 1, 77, B - 1]
-    want = attention_exact(qr[some], k[some], vt[some], True, pos, pos + 1)
-    assert ref.max_rel(out.get()[some], want) <= 2e-2
-    assert np.isfinite(out.get()).all()
+    want = attention_exact(qr, k, vt, True, pos, pos + 1)
+    assert ref.max_rel(out.get(), want) <= 2e-2
     got = dk.get()
     assert np.array_equal(np.isnan(got), np.isnan(k))
     assert ref.max_rel(np.nan_to_num(got), np.nan_to_num(k)) <= 2.0 ** -7
