@@ -227,3 +227,40 @@ def test_abi_host_paths_under_address_and_ub_sanitizers():
     out = r.stdout + r.stderr
     assert r.returncode == 0 and "SAN_OK" in r.stdout, out[-3000:]
     assert "AddressSanitizer" not in out and "runtime error" not in out, out[-3000:]
+
+
+class _Memory:
+    """Stands in for a device buffer where only the geometry of a tensor is looked at."""
+
+    def __init__(self, nbytes):
+        self.ptr, self.nbytes, self.version = 1 << 20, nbytes, 0
+
+
+def test_reshapes_check_sizes():
+    """Views of another size are refused, by reshape and by the layers' own reshapes; a residual of
+    another size too (its rows would be read past their end)."""
+    import layers
+    import tl_hip as xp
+    t = xp.DeviceTensor((2, 3, 8), "fp32", buf=_Memory(192))
+    assert t._rows().shape == (6, 8) and t.reshape(-1, 24).nrows == 2
+    for shape, rows, cols in (((2, 3, 4), 6, 4), ((5, 8), 5, 8), ((2, 4, 8), 8, 8)):
+        with pytest.raises(ValueError):
+            t._reshaped(shape, rows, cols)
+        with pytest.raises(ValueError):
+            t.reshape(shape)
+    assert layers._residual_rows(t, 6, 8).shape == (6, 8)
+    assert layers._residual_rows(t, 12, 4).shape == (12, 4)
+    for rows, cols in ((7, 8), (5, 8), (6, 16)):
+        with pytest.raises(ValueError):
+            layers._residual_rows(t, rows, cols)
+    padded = xp.DeviceTensor((6, 4), "fp32", pitch=8, buf=_Memory(192))
+    with pytest.raises(ValueError):
+        layers._residual_rows(padded, 3, 8)
+
+
+@pytest.mark.parametrize("shape,to,rows", [((0, 5), (0, 3, 5), 0), ((3, 0), (7, 0), 7), ((2, 0), (0,), 1),
+                                           ((1, 1), (), 1), ((), (1, 1), 1), ((4, 6), (2, 2, 6), 4)])
+def test_reshape_geometry(shape, to, rows):
+    import tl_hip as xp
+    t = xp.DeviceTensor(shape, "fp32", buf=_Memory(96)).reshape(to)
+    assert (t.shape, t.nrows, t.ncols) == (to, rows, to[-1] if to else 1)

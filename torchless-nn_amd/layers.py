@@ -92,6 +92,13 @@ def _prenorm(x2d, prenorm, w_dtype):
     return prenorm.output, None
 
 
+def _residual_rows(residual, M, C):
+    """A residual of M rows of C (None: none) as a 2-d tensor."""
+    if residual is None:
+        return None
+    return residual._rows() if (residual.nrows, residual.ncols) == (M, C) else residual.reshape(M, C)
+
+
 def linear(x2d, w, bias=None, act=xp.TL_ACT_NONE, residual=None, out=None, qkv=None,
            family="gemm_mfma", prenorm=None):
     """y = act(x2d @ w + bias) (+ residual), x2d [M, K], w [K, N] (reference `x @ W + b`).
@@ -243,8 +250,8 @@ class MultiHeadAttention(Layer):
         self.heads_out = heads
 
         out = linear(heads._rows(), self.out_weights, self.out_bias,
-                     residual=(residual._rows() if residual is not None else None))
-        self.output = out._reshaped((B, T, C), C)
+                     residual=_residual_rows(residual, B * T, C))
+        self.output = out._reshaped((B, T, C), B * T, C)
         return self.res_dropout.forward(self.output)
 
     def _forward_cached(self, input, residual, cache, layer, pos0):
@@ -275,8 +282,8 @@ class MultiHeadAttention(Layer):
                                                  divisor, pos0)
         self.heads_out = heads
         out = linear(heads._rows(), self.out_weights, self.out_bias,
-                     residual=(residual._rows() if residual is not None else None))
-        self.output = out._reshaped((B, T, C), C)
+                     residual=_residual_rows(residual, B * T, C))
+        self.output = out._reshaped((B, T, C), B * T, C)
         return self.res_dropout.forward(self.output)
 
     def _unfused(self, q, k, vt, B, T, C, H, D, dt, divisor):
@@ -336,8 +343,8 @@ class TransformerFeedForward(Layer):
             h = self.activation.forward(linear(x2, self.weights1, self.bias1))
         self.hidden_output = h
         y = linear(h, self.weights2, self.bias2,
-                   residual=(residual._rows() if residual is not None else None))
-        self.output = self.dropout.forward(y._reshaped(shape, C))
+                   residual=_residual_rows(residual, input.nrows, C))
+        self.output = self.dropout.forward(y._reshaped(shape, input.nrows, C))
         return self.output
 
     def set_eval(self, eval_mode):

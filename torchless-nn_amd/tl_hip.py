@@ -392,15 +392,16 @@ class DeviceTensor:
 
     def _rows(self):
         """The same rows as a 2-d tensor."""
-        return self._reshaped((self.nrows, self.ncols), self.ncols)
+        return self._reshaped((self.nrows, self.ncols), self.nrows, self.ncols)
 
-    def _reshaped(self, shape, ncols):
-        """The same elements under a shape of the same size (rows of the same pitch, or a
-        contiguous tensor's)."""
+    def _reshaped(self, shape, nrows, ncols):
+        """The same elements under `shape`, a tuple of ints with `nrows` rows of `ncols` (rows of
+        the same pitch, or a contiguous tensor's)."""
+        if nrows * ncols != self.size:
+            raise ValueError(f"cannot reshape {self.shape} into {shape}")
         t = object.__new__(DeviceTensor)
         t.shape, t.dtype, t.buf, t.offset, t.ptr = shape, self.dtype, self.buf, self.offset, self.ptr
-        t.size, t.ncols, t._aux = self.size, ncols, None
-        t.nrows = self.nrows if ncols == self.ncols else _prod(shape[:-1])
+        t.size, t.nrows, t.ncols, t._aux = self.size, nrows, ncols, None
         t.pitch = self.pitch if ncols == self.ncols else ncols
         return t
 
@@ -511,12 +512,12 @@ class DeviceTensor:
             i = shape.index(-1)
             rest = _prod(shape[:i]) * _prod(shape[i + 1:])
             shape = shape[:i] + (self.size // rest if rest else 0,) + shape[i + 1:]
-        if _prod(shape) != self.size:
+        nrows, ncols = _prod(shape[:-1]), shape[-1] if shape else 1
+        if nrows * ncols != self.size:
             raise ValueError(f"cannot reshape {self.shape} into {shape}")
-        ncols = shape[-1] if shape else 1
         if not (shape and self.shape and ncols == self.ncols) and not self.contiguous:
             raise ValueError("reshape of a padded tensor must keep the last dimension")
-        return self._reshaped(shape, ncols)
+        return self._reshaped(shape, nrows, ncols)
 
     def fill(self, value):
         if not self.contiguous:
