@@ -4,6 +4,8 @@ cores (gemm_split.hip), against float64 sums of the same inputs.
 Bars: fp32 max_rel 2e-6 sqrt(K / 256) + 2e-6 (fp32 sums of K terms: K 2^-24 at worst, sqrt(K)
 2^-24 in practice; activations and the output add a few ulps); bf16 outputs are rounded once,
 so max_rel 2^-8 plus the fp32 part, doubled."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -19,6 +21,31 @@ def xp():
     import tl_hip
     tl_hip.ctx()
     return tl_hip
+
+
+class _Rows(ctypes.Structure):
+    _fields_ = [("tile", ctypes.c_int), ("splits", ctypes.c_int), ("us", ctypes.c_float)]
+
+
+class _Split(ctypes.Structure):
+    _fields_ = [("tile", ctypes.c_int), ("full", ctypes.c_int), ("splits", ctypes.c_int),
+                ("us", ctypes.c_float)]
+
+
+def plan(xp, dt, M, N, K, cus=256):
+    """What tl_gemm makes of an unbatched [M, K] x [N, K] product with a plain tile hint: ("rows",
+    tile, splits), ("split", tile, whole tiles, splits), or None for the other kernels."""
+    def call(symbol, result):
+        f = getattr(xp.load_library(), symbol)
+        f.restype, f.argtypes = result, [ctypes.c_int64] * 3 + [ctypes.c_int]
+        return f(M, N, K, cus)
+    if dt == "bf16":
+        r = call("_ZN2tl14gemm_rows_planEllli", _Rows)
+        return ("rows", r.tile, r.splits) if r.tile >= 0 else None
+    r, s = call("_ZN2tl18gemm_rows_plan_f32Ellli", _Rows), call("_ZN2tl15gemm_split_planEllli", _Split)
+    if r.tile >= 0 and (s.tile < 0 or r.us <= s.us):
+        return ("rows", r.tile, r.splits)
+    return ("split", s.tile, s.full, s.splits) if s.tile >= 0 else None
 
 
 def bar(dt, K):
@@ -100,13 +127,14 @@ def test_few_tiles_gated(xp, mnk):
 
 # whole tiles only, a last round split over K, everything split, tails of one row and column,
 # one K step
-SPLIT = [(2048, 2048, 256), (2305, 1025, 96), (4000, 2304, 768), (1281, 769, 3072), (1025, 2049, 32),
-         (13050, 256, 256)]
+SPLIT = [(2048, 2048, 256), (1281, 3073, 96), (4000, 2304, 768), (1281, 769, 3072), (4097, 1025, 32),
+         (13050, 256, 256), (6145, 1025, 32), (12289, 513, 64)]
 
 
 @pytest.mark.parametrize("mnk", SPLIT)
 def test_fp32_pieces(xp, mnk):
     M, N, K = mnk
+    assert plan(xp, "fp32", M, N, K)[0] == "split"
     a, w, bias, res = inputs(xp, "fp32", M, N, K)
     da, dw, db, dres = (xp.array(t, dtype="fp32") for t in (a, w, bias, res))
     y = a.astype(np.float64) @ w.astype(np.float64).T
@@ -120,19 +148,68 @@ def test_fp32_pieces(xp, mnk):
     assert ref.max_rel(out.get(), y + bias + res) <= bar("fp32", K)
 
 
-@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
-def test_fp32_pieces_scales(xp, scale):
-    """Operands far from 1: sums as close as at scale 1 (the smallest are redone in fp32)."""
-    M, N, K = 1100, 1100, 128
-    a, w, _, _ = inputs(xp, "fp32", M, N, K)
-    a = (a * F32(scale)).astype(F32)
+# one product per form of gemm_split_kernel: small tiles, large tiles with the last ones split over K
+FORMS = [(2048, 2048, 256), (4000, 2304, 768)]
+
+
+def fp32_product(xp, a, w, tile="auto"):
+    (M, K), N = a.shape, w.shape[0]
+    if tile == "auto":
+        assert plan(xp, "fp32", M, N, K)[0] == "split"
     out = xp.empty((M, N), "fp32")
     xp.gemm(xp.array(a, dtype="fp32"), xp.array(w, dtype="fp32"), M=M, N=N, K=K, lda=K, ldb=K,
-            b_layout=xp.TL_B_NK, C=out, ldc=N)
-    assert ref.max_rel(out.get(), a.astype(np.float64) @ w.astype(np.float64).T) <= bar("fp32", K)
+            b_layout=xp.TL_B_NK, C=out, ldc=N, tile=tile)
+    return out.get()
 
 
-@pytest.mark.parametrize("mnk", [(1100, 1100, 128), (2305, 1025, 1024)])
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("ea,ew", [(-120, 100), (-124, 123), (-136, 115), (-136, 0)])
+@pytest.mark.parametrize("mnk", FORMS)
+def test_fp32_pieces_tiny_beside_huge(xp, mnk, ea, ew, swap):
+    """Tiny elements, whose pieces are lost in part or whole, times huge ones (ordinary sums), and
+    times ordinary ones (sums of no pieces at all): as close as the fp32 MFMA, whose sums of K
+    products of normal operands are within the bar of float64."""
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, "fp32", M, N, K)
+    w *= F32(K ** 0.5)
+    a, w = np.ldexp(a, ew if swap else ea), np.ldexp(w, ea if swap else ew)
+    got, old = fp32_product(xp, a, w), fp32_product(xp, a, w, tile="128x128")
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    floor = K * 2.0 ** -149 / np.abs(want).max()  # of sums that are fp32 denormals
+    assert ref.max_rel(got, old) <= 2 * bar("fp32", K) + floor
+    if ea > -126:
+        assert ref.max_rel(got, want) <= bar("fp32", K) + floor
+
+
+@pytest.mark.parametrize("mnk", FORMS)
+def test_fp32_pieces_mixed_magnitudes(xp, mnk):
+    """One tiny row against one huge column, the rest ordinary, with zero rows: every row and every
+    column is as close to float64 as among its own kind."""
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, "fp32", M, N, K)
+    a[7], w[11] = np.ldexp(a[7], -122), np.ldexp(w[11], 120)
+    a[64:70], w[100] = 0, 0
+    got = fp32_product(xp, a, w)
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    assert abs(got[7, 11] / want[7, 11] - 1) <= 1e-4  # one sum, which may cancel
+    rows, cols = np.arange(M) != 7, np.arange(N) != 11
+    for r, c in ((rows, cols), (rows, ~cols)):
+        assert ref.max_rel(got[r][:, c], want[r][:, c]) <= bar("fp32", K)
+    assert np.abs(got[7, cols] - want[7, cols]).max() <= K * 2.0 ** -149 + 1e-6 * np.abs(want[7, cols]).max()
+    assert not got[64:70].any() and not got[:, 100].any()
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
+@pytest.mark.parametrize("mnk", FORMS)
+def test_fp32_pieces_scales(xp, mnk, scale):
+    """Operands far from 1: sums as close as at scale 1 (the smallest are redone in fp32)."""
+    M, N, K = mnk
+    a, w, _, _ = inputs(xp, "fp32", M, N, K)
+    a = (a * F32(scale)).astype(F32)
+    assert ref.max_rel(fp32_product(xp, a, w), a.astype(np.float64) @ w.astype(np.float64).T) <= bar("fp32", K)
+
+
+@pytest.mark.parametrize("mnk", [(2048, 2048, 128), (2305, 1025, 1024), (4000, 2304, 768)])
 def test_fp32_pieces_not_finite(xp, mnk):
     """Infinities, NaN and values past bf16's largest give what fp32 sums give, in their rows
     and columns alone; a denormal row gives what the fp32 MFMA kernel gives."""
@@ -142,11 +219,7 @@ def test_fp32_pieces_not_finite(xp, mnk):
     w[10, 9], w[600, 1] = np.inf, np.nan
     w[20] *= F32(1e-3)  # 3.4e38 stays finite there
     a[1000] = F32(1e-40)
-    out, old = xp.empty((M, N), "fp32"), xp.empty((M, N), "fp32")
-    for o, tile in ((out, "auto"), (old, "128x128")):  # a named tile keeps the fp32 MFMA kernel
-        xp.gemm(xp.array(a, dtype="fp32"), xp.array(w, dtype="fp32"), M=M, N=N, K=K, lda=K, ldb=K,
-                b_layout=xp.TL_B_NK, C=o, ldc=N, tile=tile)
-    got = out.get()
+    got, old = fp32_product(xp, a, w), fp32_product(xp, a, w, tile="128x128")  # the fp32 MFMA kernel
     with np.errstate(all="ignore"):
         want = a.astype(np.float64) @ w.astype(np.float64).T
         want[np.abs(want) > 3.5e38] *= np.inf
@@ -161,7 +234,7 @@ def test_fp32_pieces_not_finite(xp, mnk):
     assert ref.max_rel(np.where(ok, got, 0)[rows], np.where(ok, want, 0)[rows]) <= bar("fp32", K)
     assert ref.max_rel(np.where(ok, got, 0)[900], np.where(ok, want, 0)[900]) <= bar("fp32", K)
     with np.errstate(all="ignore"):
-        low = np.where(ok, got - old.get(), 0)[1000]
+        low = np.where(ok, got - old, 0)[1000]
     assert np.abs(low).max() <= K * 2.0 ** -149
 
 

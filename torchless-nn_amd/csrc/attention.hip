@@ -1644,7 +1644,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         y[v] = (o[rt][t][v] * f1 + w[(2 + 4 * t + v) * 64] * f2) * inv;
-        bad = bad || pieces_doubtful(y[v]);
+        bad = bad || (y[v] != 0.f && pieces_doubtful(y[v], 0x1p-60f));
       }
       if (qpos < p.Tq) *reinterpret_cast<f32x4*>(oh + (int64_t)qpos * p.ld_out + 16 * t + 4 * fg) = y;
     }

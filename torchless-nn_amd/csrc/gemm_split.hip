@@ -6,10 +6,12 @@
 // taken (fp32_pieces.hpp), with fewer fp32 roundings than the fp32 MFMA's (6 accumulating
 // instructions per 32 of K instead of 8).
 //
-// Operands the split cannot represent are recomputed: an infinity, a NaN or a value that rounds
-// past bf16's largest gives a NaN or infinite sum, operands so small that pieces underflow give
-// tiny sums. A wave that holds a sum outside [2^-60, inf) that is not 0 redoes its block with the
-// fp32 MFMA straight from memory, so such results are what gemm_mfma_f32_kernel gives.
+// What the pieces cannot represent is recomputed: an infinity, a NaN or a value that rounds past
+// bf16's largest gives a NaN or infinite sum, and parts of tiny elements that are lost matter only
+// in sums that are small beside the tile's largest element (fp32_pieces.hpp). A wave that holds a
+// nonzero sum outside [least, inf), least = max(2^-60, K 2^-96 largest), redoes its block with the
+// fp32 MFMA straight from memory, and so does one that holds a 0 whose row or column has an element
+// below 2^-63 (zeros_doubtful). Such results are what gemm_mfma_f32_kernel gives.
 //
 // Layout: K steps of 32; the fp32 elements of the next step are loaded into registers, split on
 // the vector ALUs and written as three bf16 planes [rows][32] to LDS (16-byte chunks, XOR-swizzled
@@ -19,14 +21,74 @@
 // one buffer, three workgroups per CU, whose phases overlap each other's. Bound by the matrix cores
 // and the LDS reads (24 fragments per 96 MFMAs) once the chip is full: 8192 x 50257 x 768 5801 ->
 // 3262 us (194 TFLOP/s of fp32 products, 1.16 PFLOP/s on the matrix cores), 4000 x 3072 x 768 174 ->
-// 107, 4000 x 768 x 3072 230 -> 108 us; error against 64 bits 3.0e-7 where the fp32 MFMA's is
-// 3.5e-7 (K = 768; 0.8 to 0.9 of it at every size measured, K 128 .. 4096).
+// 107, 4000 x 768 x 3072 230 -> 108 us; error against 64 bits 4.2e-7 where the fp32 MFMA's is
+// 5.0e-7 (1024 x 50257 x 768; 0.78 to 0.85 of it over 10007 to 50257 columns, K 256 .. 768). The
+// largest element and the look at the sums cost nothing that shows (before and after: 4000 x 3072 x
+// 768 123 and 123 us, 4000 x 768 x 3072 126 and 125, 2048 x 2048 x 256 23.6 and 22.3).
 #include <algorithm>
 
 #include "fp32_pieces.hpp"
 #include "gemm_split.hpp"
 
 namespace tl {
+
+// Whether one of a wave's sums that are 0 belongs to a row of A or of B with a tiny element: rows a0 + r
+// (r < 16 TM, clamped to a_last) of A, b0 + c of B, K elements each. A row of A that is all zeros
+// has sums of 0 whatever the columns hold. Wave-uniform.
+template <int TM, int TN>
+__device__ __forceinline__ bool zeros_doubtful(const f32x4 (&acc)[TM][TN], const float* A, int64_t lda, int a0, int a_last,
+                                               const float* B, int64_t ldb, int b0, int b_last, int K) {
+  const int lane = threadIdx.x & 63, fr = lane & 15;
+  auto scan = [&](const float* row, bool& tiny) {  // whether the row has a nonzero element
+    bool some = false;
+    for (int k = lane * 4; k < K; k += 256) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(row + k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        some |= x[e] != 0.f;
+        tiny |= pieces_tiny(x[e]);
+      }
+    }
+    tiny = __any(tiny);
+    return __any(some);
+  };
+  bool tiny = false;
+  uint64_t rows = 0, cols = 0;  // those with sums of 0
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    bool z = false;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) z |= acc[i][j][q] == 0.f;
+    uint64_t b = __ballot(z);
+    b |= b >> 32;
+    b |= b >> 16;
+    rows |= (b & 0xffff) << (16 * i);
+  }
+  for (uint64_t left = rows; left; left &= left - 1) {
+    const int r = __builtin_ctzll(left);
+    if (!scan(A + (int64_t)min(a0 + r, a_last) * lda, tiny)) rows &= ~(1ull << r);
+    if (tiny) return true;
+  }
+  if (!rows) return false;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bool z = false;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) z |= acc[i][j][q] == 0.f && (rows >> (16 * i + fr) & 1);
+      const uint64_t b = __ballot(z);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) cols |= (uint64_t)((b >> (16 * g) & 0xffff) != 0) << (16 * j + 4 * g + q);
+    }
+  for (; cols; cols &= cols - 1) {
+    scan(B + (int64_t)min(b0 + __builtin_ctzll(cols), b_last) * ldb, tiny);
+    if (tiny) return true;
+  }
+  return false;
+}
 
 template <typename TO, int BM, int BN, int WGM, int WGN, int NBUF>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p, float* part, int full, int splits) {
@@ -37,6 +99,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p
   static_assert(ROWS * 4 % NT == 0 && BM * 4 % NT == 0 && TM >= 1 && TN >= 1, "bad tile/thread split");
   static_assert(NBUF * 3 * PLANE * 2 <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) bf16_t S[NBUF][3 * PLANE];
+  __shared__ float wave_most[WGM * WGN];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WGN, wn = wave - wm * WGN;
@@ -99,11 +162,12 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p
   };
   // every pass of chunks shares one swizzled slot: NT / 4 rows are a multiple of 8
   const int slot = (tid >> 2) * BK + ((lc ^ ((tid >> 3) & 3)) << 3);
+  float most = 0.f;  // largest magnitude this thread has split
   auto store = [&](bf16_t* B) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       uint4 p1, p2, p3;
-      split8(raw[i], p1, p2, p3);
+      split8(raw[i], p1, p2, p3, most);
       bf16_t* dst = B + slot + i * (NT / 4) * BK;
       *reinterpret_cast<uint4*>(dst) = p1;
       *reinterpret_cast<uint4*>(dst + PLANE) = p2;
@@ -166,13 +230,30 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split_kernel(GemmParams p
 
   const int64_t mb = m0 + wm * WM + fr, nb = n0 + wn * WN;
   {
-    bool bad = false;
+    most = wave_max(most);
+    if (lane == 0) wave_most[wave] = most;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WGM * WGN; ++w) most = fmaxf(most, wave_most[w]);
+    const float least = pieces_least(most, K);
+    bool look = false, bad = false;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) bad = bad || pieces_doubtful(acc[i][j][q]);
+        for (int q = 0; q < 4; ++q) look = look || pieces_doubtful(acc[i][j][q], least);
+    if (__any(look)) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) bad = bad || (pieces_doubtful(acc[i][j][q], least) && acc[i][j][q] != 0.f);
+      if (!__any(bad))
+        bad = zeros_doubtful<TM, TN>(acc, Ab, p.lda, wm * WM, (int)min((int64_t)BM, p.M - m0) - 1, Bb, p.ldb,
+                                     wn * WN, (int)min((int64_t)BN, p.N - n0) - 1, K);
+    }
     if (__any(bad)) {  // this wave's block again on the fp32 matrix cores (see above)
       const float* Ar[TM];
       const float* Br[TN];
