@@ -333,6 +333,42 @@ def test_fp32_attention_pieces_not_finite(xp, D):
     assert ref.max_rel(got[0, :176, 4], want[0, :176, 4]) <= 4e-6
 
 
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("eq,ek", [(-122, 122), (-136, 124), (-104, 100)])
+@pytest.mark.parametrize("D", [32, 64])
+def test_fp32_attention_pieces_tiny_beside_huge(xp, D, eq, ek, swap):
+    """Tiny queries against huge keys, or the other way round: ordinary scores (their products carry
+    one rounding of each operand, which the inputs already hold), so ordinary outputs."""
+    B, H, T = 2, 2, 150
+    rng = np.random.default_rng(D + 200 + eq)
+    q, k, vt = (rng.standard_normal(s, dtype=F32) for s in ((B, H, T, D), (B, H, T + 2, D), (B, H, D, T + 2)))
+    q, k = np.ldexp(q, ek if swap else eq), np.ldexp(k, eq if swap else ek)
+    out = xp.empty((B, T, H * D), "fp32")
+    xp.attention(*(xp.array(t, dtype="fp32") for t in (q, k, vt)), out, n_heads_q=H, n_heads_kv=H,
+                 divisor=float(F32(D ** 0.5)), causal=True, offset=0, seq_k=T)
+    assert ref.max_rel(out.get(), attention_exact(q, k, vt, True, 0, T)) <= 4e-6
+
+
+@pytest.mark.parametrize("D", [32, 64])
+def test_fp32_attention_pieces_tiny_probabilities(xp, D):
+    """Values that are huge where the probabilities are tiny and 0 at the key that takes them all;
+    scores of up to 124 in log2 units carry 2^-17 of themselves into such a probability. And values
+    that are all tiny: outputs within fp32's denormal steps."""
+    B, H, T = 1, 2, 144
+    rng = np.random.default_rng(D)
+    q, k = (rng.standard_normal((B, H, T, D), dtype=F32) * F32(0.05) for _ in range(2))
+    vt = np.ldexp(rng.standard_normal((B, H, D, T), dtype=F32), 122)
+    q[..., 0], k[..., 0], k[:, :, 0, 0] = 1, 0, F32(119 * np.log(2) * D ** 0.5)
+    vt[..., 0] = 0
+    vt[0, 1] = np.ldexp(rng.standard_normal((D, T), dtype=F32), -136)
+    out = xp.empty((B, T, H * D), "fp32")
+    xp.attention(*(xp.array(t, dtype="fp32") for t in (q, k, vt)), out, n_heads_q=H, n_heads_kv=H,
+                 divisor=float(F32(D ** 0.5)), causal=False, offset=0, seq_k=T)
+    got, want = out.get(), attention_exact(q, k, vt, False, 0, T)
+    assert ref.max_rel(got[..., :D], want[..., :D]) <= 2.0 ** -13
+    assert np.abs(got[..., D:] - want[..., D:]).max() <= 4 * 2.0 ** -149
+
+
 # 256x256 tiles that fill the chip: one to many K steps (odd and even counts), remainders of rows
 # and columns, more than one round, a K beyond the late-load form's
 @pytest.mark.parametrize("mnk", [(8192, 2048, 256), (8192, 2048, 320), (4096, 4096, 384),

@@ -1332,12 +1332,16 @@ __global__ __launch_bounds__(256) void attention_fwd_f32_kernel(AttnParams p) {
 // bf16 planes each (one 48 KB buffer at head dim 64: three workgroups per CU, whose loads,
 // splitting and MFMAs overlap each other's). Heavy causal blocks are dispatched first.
 //
-// A wave whose merged outputs are not all finite, or tiny, redoes its 32 rows with the fp32 MFMA
-// straight from memory (attend_rows_f32), so infinities, NaN and tiny operands give what fp32 sums
-// give.
+// What the pieces cannot represent (fp32_pieces.hpp) is redone, a wave's 32 rows at a time, with the
+// fp32 MFMA straight from memory (attend_rows_f32): outputs that are not finite; outputs that are
+// small beside the largest value (a tiny probability may have lost a part, which counts beside a
+// huge value; probabilities reach 2^8 before they are divided by a sum of at least 2^-8); outputs
+// of 0 over values of which some are tiny; and every row when the largest query or key is so large
+// that a lost part of a tiny partner could move a score by 2^-30.
 //
 // GPT-2-small heads, 4 x 1000 tokens: 110 -> 63 us (98 TFLOP/s of fp32 products); 8 x 1024: 150 ->
-// 104; error against 64 bits 2.0e-7 (fp32 MFMA 3.3e-7). Bound by issue: the splitting and the
+// 104 (the looks at magnitudes and outputs cost nothing that shows: 106 without them, 104 with);
+// error against 64 bits 2.0e-7 (fp32 MFMA 3.3e-7). Bound by issue: the splitting and the
 // softmax take as many cycles as the MFMAs, at two waves per SIMD (213 registers). Held to 168 for
 // three it spills and took 80 us, without the register prefetch 70; more independent sums between
 // two products of one changed nothing.
@@ -1411,6 +1415,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
   constexpr int KPL = BKV * D, VPL = D * BKV;            // elements of a plane
   static_assert(D == 32 || D == 64, "head dims 32 and 64");
   __shared__ __attribute__((aligned(16))) bf16_t S[3 * KPL + 3 * VPL];
+  __shared__ float wave_most[2][4];
   bf16_t* Ks = S;
   bf16_t* Vs = S + 3 * KPL;
 
@@ -1459,6 +1464,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
   auto kslot = [&](int r, int c) {  // 16-byte chunk c of a K row, swizzled
     return r * D + ((c ^ (KCH == 8 ? r & 7 : (r >> 1) & 3)) << 3);
   };
+  float most_qk = 1.f, most_v = 0.f;  // largest magnitudes this thread has split
   auto store_chunk = [&](int kv0) {
     if (kv0 + BKV > p.Tk) {  // values past Tk (never written) are zeroed: 0 * NaN is not 0
 #pragma unroll
@@ -1471,7 +1477,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
     for (int i = 0; i < KU; ++i) {
       const int u = i * 256 + tid;
       uint4 a, b2, c;
-      split8(rk[i], a, b2, c);
+      split8(rk[i], a, b2, c, most_qk);
       bf16_t* dst = Ks + kslot(u / KCH, u % KCH);
       *reinterpret_cast<uint4*>(dst) = a;
       *reinterpret_cast<uint4*>(dst + KPL) = b2;
@@ -1481,7 +1487,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
     for (int i = 0; i < VU; ++i) {  // two 4-key groups, in the key order of the P.V operand
       const int u = i * 256 + tid, r = u >> 3, g = 2 * (u & 7);
       uint4 a, b2, c;
-      split8(rv[i], a, b2, c);
+      split8(rv[i], a, b2, c, most_v);
       bf16_t* lo = Vs + r * BKV + vperm_slot(g, r);
       bf16_t* hi = Vs + r * BKV + vperm_slot(g + 1, r);
       *reinterpret_cast<uint2*>(lo) = make_uint2(a.x, a.y);
@@ -1505,7 +1511,7 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = qrow[32 * ks + e];
       uint4 a, b2, c;
-      split8(x, a, b2, c);
+      split8(x, a, b2, c, most_qk);
       qf[rt][ks][0] = __builtin_bit_cast(bf16x8, a);
       qf[rt][ks][1] = __builtin_bit_cast(bf16x8, b2);
       qf[rt][ks][2] = __builtin_bit_cast(bf16x8, c);
@@ -1612,6 +1618,12 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
   // merge the two key halves of each row group: the second leaves its state in LDS
   float* red = reinterpret_cast<float*>(S) + rg * (2 * (DT * 4 + 2) * 64) + lane;
   static_assert(2 * 2 * (DT * 4 + 2) * 64 * 4 <= (int)sizeof(S), "merge space");
+  most_qk = wave_max(most_qk);
+  most_v = wave_max(most_v);
+  if (lane == 0) {
+    wave_most[0][wave] = most_qk;
+    wave_most[1][wave] = most_v;
+  }
   __syncthreads();
   if (kh2 == 1) {
 #pragma unroll
@@ -1627,7 +1639,14 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
   }
   __syncthreads();
   if (kh2 == 1) return;
-  bool bad = false;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    most_qk = fmaxf(most_qk, wave_most[0][w]);
+    most_v = fmaxf(most_v, wave_most[1][w]);
+  }
+  const float least = pieces_least(0x1p+8f * most_v, p.Tk);
+  bool bad = !((float)D * (most_qk * 0x1p-124f) * p.scale_log2 < 0x1p-30f);
+  bool look = false;
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
     const float* w = red + rt * (DT * 4 + 2) * 64;
@@ -1644,9 +1663,30 @@ __global__ __launch_bounds__(256) void attention_fwd_pieces_kernel(AttnParams p,
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         y[v] = (o[rt][t][v] * f1 + w[(2 + 4 * t + v) * 64] * f2) * inv;
-        bad = bad || (y[v] != 0.f && pieces_doubtful(y[v], 0x1p-60f));
+        look = look || pieces_doubtful(y[v], least);
       }
+      o[rt][t] = y;
       if (qpos < p.Tq) *reinterpret_cast<f32x4*>(oh + (int64_t)qpos * p.ld_out + 16 * t + 4 * fg) = y;
+    }
+  }
+  if (__any(look)) {
+    uint64_t zeros = 0;  // head dims with an output of 0: their values once more, for tiny ones
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float y = o[rt][t][v];
+          bad = bad || (y != 0.f && pieces_doubtful(y, least));
+          const uint64_t z = __ballot(y == 0.f);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) zeros |= (uint64_t)((z >> (16 * g) & 0xffff) != 0) << (16 * t + 4 * g + v);
+        }
+    for (; zeros; zeros &= zeros - 1) {
+      const float* vrow = vh + (int64_t)__builtin_ctzll(zeros) * p.Lk;
+#pragma unroll 4
+      for (int kv = lane; kv < kv_end; kv += 64) bad |= pieces_tiny(vrow[kv]);
     }
   }
   if (__any(bad)) {
