@@ -264,3 +264,70 @@ def test_reshape_geometry(shape, to, rows):
     import tl_hip as xp
     t = xp.DeviceTensor(shape, "fp32", buf=_Memory(96)).reshape(to)
     assert (t.shape, t.nrows, t.ncols) == (to, rows, to[-1] if to else 1)
+
+
+class _FakeContext:
+    """A context whose graphs launch nothing; `capture` is set as xp.capture sets it."""
+
+    class lib:
+        @staticmethod
+        def tl_graph_launch(handle, graph):
+            return 0
+
+        tl_graph_destroy = tl_graph_launch
+
+    handle, capture = 1, None
+
+
+def test_graphs_keep_and_remake_the_copies_they_read(monkeypatch):
+    """A copy that a captured call found current keeps its address and is made again before a launch
+    when a source was written, whether or not an eager call did so first; a copy that it did not
+    find current is made inside the capture, once, and leaves the kept one alone."""
+    import tl_hip as xp
+    c = _FakeContext()
+    monkeypatch.setattr(xp, "_ctx", c)
+    source, slots, made = xp.DeviceTensor((4, 4), "fp32", buf=_Memory(64)), {}, []
+
+    def make(out):
+        made.append(out)
+        return out if out is not None else object()
+
+    def copy():
+        return xp.derived(slots, None, source._version, (source,), make, copy)
+
+    class Open:
+        def __init__(self):
+            self._derived, self._recorded = {}, {}
+
+    def captured():
+        c.capture = cap = Open()
+        first, second = copy(), copy()
+        c.capture = None
+        assert first is second
+        return first, xp.Graph(7, cap._derived.values())
+
+    source._version += 1
+    recorded, graph = captured()  # nothing kept yet
+    assert made == [None] and not slots
+    graph.launch()
+    kept = copy()
+    assert kept is not recorded and made == [None, None]
+    read, graph = captured()
+    assert read is kept and len(made) == 2
+    graph.launch()
+    assert len(made) == 2  # still current
+    source._version += 1
+    graph.launch()
+    graph.launch()
+    assert made[2:] == [kept]  # in place, once
+    source._version += 1
+    assert copy() is kept and made[2:] == [kept] * 2
+    graph.launch()
+    assert len(made) == 4
+    source._version += 1
+    c.capture = Open()
+    assert copy() is not kept  # written since: the capture records the making
+    c.capture = None
+    graph.launch()
+    assert made[-1] is kept and copy() is kept
+    graph.destroy()

@@ -358,3 +358,44 @@ def test_captured_forward_matches_predict(tl, dt):
     with pytest.raises(ValueError):
         fwd(xp.array(first[:2]))
     fwd.destroy()
+
+
+@pytest.mark.parametrize("eager_first", [True, False])
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
+def test_replays_follow_rewritten_weights(tl, dt, eager_first):
+    """A captured product of few rows (it reads a packed copy of its weight) after the weight was
+    written: replays use the new weight, with and without an eager call in between and with the
+    pool's blocks handed out to others; and captured before any eager call, where later eager calls
+    get a copy of their own."""
+    xp, layers = tl["xp"], tl["layers"]
+    rng = np.random.default_rng(7)
+    M, K, N = 24, 768, 384
+    x = xp.array(rng.standard_normal((M, K)).astype(F32), dtype=dt)
+    w = xp.array(rng.standard_normal((K, N)).astype(F32), dtype=dt)
+    tl["backend"].set_float_type(dt)
+    norm = layers.RMSNorm(K, gamma_offset=1.0) if dt == "bf16" else None
+    tl["backend"].set_float_type("fp32")
+    call = lambda: layers.linear(x, w, prenorm=norm)  # noqa: E731
+    if eager_first:
+        call()
+    with xp.capture() as g:
+        y = call()
+    for step in range(4):
+        if step:
+            w.set(rng.standard_normal((K, N)).astype(F32))
+        if step == 3 and norm is not None:
+            norm.gamma.fill(0.5)
+        if step == 2:
+            call()
+        junk = [xp.array(np.full((K, N), 1e3, F32), dtype=dt) for _ in range(3)]
+        g.launch()
+        got = y.get()
+        xp.synchronize()
+        assert np.abs(got - call().get()).max() <= np.abs(got).max() * (1e-2 if dt == "bf16" else 1e-5), step
+        want = x.get().astype(np.float64)
+        if norm is not None:
+            want = want / np.sqrt((want ** 2).mean(-1, keepdims=True) + 1e-6) * (1 + norm.gamma.get())
+        want = want @ w.get().astype(np.float64)
+        assert np.abs(got - want).max() <= np.abs(want).max() * (2e-2 if dt == "bf16" else 1e-5), step
+        del junk
+    g.destroy()

@@ -12,8 +12,9 @@ reference; every forward is a handful of libtl kernel launches on one HIP stream
   LayerNorm / RMSNorm       -> one row kernel each
 
 The MFMA GEMMs read a weight in a K-contiguous copy ([out, in]) that is packed on the
-device the first time the weight is used and again after its buffer has been written (by
-`set`, `fill` or any kernel writing into any view of it). bf16 weights always take that copy;
+device the first time the weight is used and again, in place, after its buffer has been written
+(by `set`, `fill` or any kernel writing into any view of it); a captured graph that reads the copy
+has that done before a launch. bf16 weights always take that copy;
 fp32 weights take it for products the matrix-core kernels run (K % 32 == 0; or K % 4 == 0 and
 either at least 128 output tiles of 128x128 or K <= 1024 with at least 8 tiles of 64x64), which
 doubles their HBM use, and are read in place by the fp32 VALU GEMM otherwise.
@@ -35,19 +36,24 @@ def _round_up(n, m):
 
 
 def _packed_nk(w, prenorm=None):
-    """[K, N] weight -> [N, K] (K-contiguous) copy for the MFMA GEMM, cached on the
+    """[K, N] weight -> [N, K] (K-contiguous) copy for the MFMA GEMM, kept on the
     weight until its contents change. With `prenorm` (the RMSNorm layer that feeds the
     product) its gain is folded in: B[n, k] = w[k, n] * (gamma_offset + gamma[k])."""
-    key = ((w._version,) if prenorm is None else
-           (w._version, prenorm.gamma._version, prenorm.gamma_offset))
-    if w._aux is not None and w._aux[0] == key:
-        return w._aux[1]
+    if w._aux is None:
+        w._aux = {}
     if prenorm is None:
-        packed = xp.transpose2d(w)
-    else:
-        packed = xp.transpose2d_gain(w, prenorm.gamma, prenorm.gamma_offset)
-    w._aux = (key, packed)
-    return packed
+        kept = w._aux.get(None)
+        if kept is not None and kept[0] == w.buf.version and xp._ctx.capture is None:
+            return kept[1]
+    K = w.shape[0]
+    if prenorm is None:
+        return xp.derived(w._aux, None, w.buf.version, (w,),
+                          lambda out: xp.transpose2d(w, out=out, ldy=K), lambda: _packed_nk(w))
+    gamma, offset = prenorm.gamma, prenorm.gamma_offset
+    key = (w.buf.version, gamma.buf.version, offset)
+    return xp.derived(w._aux, gamma, key, (w, gamma),
+                      lambda out: xp.transpose2d_gain(w, gamma, offset, out=out, ldy=K),
+                      lambda: _packed_nk(w, prenorm))
 
 
 def _warm(rows, *weights):
@@ -85,10 +91,9 @@ def _prenorm(x2d, prenorm, w_dtype):
     if M <= 16 and K % 8 == 0 and x2d.pitch % 8 == 0 and x2d.ptr % 16 == 0:
         prenorm.output = None
         return x2d, float(prenorm.eps)
-    key = (K, x2d.dtype.name)
-    if key not in _UNIT_GAIN:
-        _UNIT_GAIN[key] = xp.zeros((K,), x2d.dtype)
-    prenorm.output = xp.rmsnorm(x2d, _UNIT_GAIN[key], prenorm.eps, 1.0)
+    unit = xp.derived(_UNIT_GAIN, (K, x2d.dtype.name), 0, (), lambda _: xp.zeros((K,), x2d.dtype),
+                      lambda: None)
+    prenorm.output = xp.rmsnorm(x2d, unit, prenorm.eps, 1.0)
     return prenorm.output, None
 
 
@@ -96,7 +101,9 @@ def _residual_rows(residual, M, C):
     """A residual of M rows of C (None: none) as a 2-d tensor."""
     if residual is None:
         return None
-    return residual._rows() if (residual.nrows, residual.ncols) == (M, C) else residual.reshape(M, C)
+    if residual.nrows == M and residual.ncols == C:
+        return residual._rows()
+    return residual.reshape(M, C)
 
 
 def linear(x2d, w, bias=None, act=xp.TL_ACT_NONE, residual=None, out=None, qkv=None,
@@ -114,14 +121,11 @@ def linear(x2d, w, bias=None, act=xp.TL_ACT_NONE, residual=None, out=None, qkv=N
     if qkv is None and out is None:
         out = xp.DeviceTensor._alloc((M, N), x2d.dtype, M, N)
     # bf16 always; fp32 when a matrix-core kernel takes the product, which reads B as [N, K]:
-    # K % 4 == 0 and either at least 128 output tiles of 128x128 or K <= 1024 with 8 or more
-    # 64x64 tiles, or any other K % 32 == 0 (24 x 768 x 3072: 37 us on the vector ALUs, 14 us
-    # packed). A weight not packed yet is not packed for the last kind inside a graph capture,
-    # where the copy would be recorded instead of made.
-    if w.dtype is xp.bfloat16 or (K % 4 == 0 and (-(-M // 128) * -(-N // 128) >= 128 or
-                                                  (K <= 1024 and -(-M // 64) * -(-N // 64) >= 8))) or (
-            K % 32 == 0 and w.dtype is xp.float32 and
-            (not xp.capturing() or (w._aux is not None and w._aux[0] == (w._version,)))):
+    # K % 32 == 0 (24 x 768 x 3072: 37 us on the vector ALUs, 14 us packed), or K % 4 == 0 and
+    # either at least 128 output tiles of 128x128 or K <= 1024 with 8 or more 64x64 tiles
+    if w.dtype is xp.bfloat16 or (K % 32 == 0 and w.dtype is xp.float32) or (
+            K % 4 == 0 and (-(-M // 128) * -(-N // 128) >= 128 or
+                            (K <= 1024 and -(-M // 64) * -(-N // 64) >= 8))):
         B, ldb, layout = _packed_nk(w, fold), K, xp.TL_B_NK
     else:
         B, ldb, layout = w, w.pitch, xp.TL_B_KN
@@ -659,25 +663,28 @@ class GeGLUFeedForward(Layer):
         self.down_weights = backend.init_random_tensor((F, C), divisor=F ** 0.5)
         for w in (self.gate_weights, self.up_weights, self.down_weights):
             self.register_param(w)
-        self._pack = None
+        self._pack = {}
 
     def _packed(self, prenorm=None):
         """Gate and up weights interleaved as [2F, C] rows (gate f, up f), with the gain of
         `prenorm` (the RMSNorm feeding the FFN) folded in when given."""
         g, u = self.gate_weights, self.up_weights
-        key = ((g._version, u._version) if prenorm is None else
-               (g._version, u._version, prenorm.gamma._version, prenorm.gamma_offset))
-        if self._pack is None or self._pack[0] != key:
+        gamma, offset = (None, 0.0) if prenorm is None else (prenorm.gamma, prenorm.gamma_offset)
+
+        def make(packed):
             C, F = g.shape
-            packed = xp.empty((2 * F, C), g.dtype)
+            if packed is None or packed.shape != (2 * F, C) or packed.dtype is not g.dtype:
+                packed = xp.empty((2 * F, C), g.dtype)
             for w, at in ((g, 0), (u, C)):
-                if prenorm is None:
+                if gamma is None:
                     xp.transpose2d(w, out=packed, out_offset=at, ldy=2 * C)
                 else:
-                    xp.transpose2d_gain(w, prenorm.gamma, prenorm.gamma_offset, out=packed,
-                                        out_offset=at, ldy=2 * C)
-            self._pack = (key, packed)
-        return self._pack[1]
+                    xp.transpose2d_gain(w, gamma, offset, out=packed, out_offset=at, ldy=2 * C)
+            return packed
+
+        sources = (g, u) if gamma is None else (g, u, gamma)
+        return xp.derived(self._pack, gamma, (*(t._version for t in sources), offset), sources, make,
+                          lambda: self._packed(prenorm))
 
     def forward(self, input):
         return self._forward(input, None)

@@ -264,7 +264,7 @@ class Context:
         self.device = device
         self.lib = lib
         self.malloc, self.free = lib.tl_malloc, lib.tl_free
-        self.capturing = False  # between tl_graph_begin and tl_graph_end
+        self.capture = None  # the open `capture`, between tl_graph_begin and tl_graph_end
 
     def sync(self):
         check(self.lib.tl_sync(self.handle))
@@ -1066,15 +1066,30 @@ class Graph:
     launch. Use as `with xp.capture() as g: <calls>`, then `g.launch()`. The calls in the
     block are recorded, not run; tensors allocated inside are written on every replay."""
 
-    def __init__(self, handle):
+    def __init__(self, handle, derived=()):
         self._handle, self._ctx = handle, ctx()
+        # copies that the captured calls read (a packed weight): how each is brought up to date, and
+        # the version of every buffer they are made from when that was last done
+        self._remake = [remake for remake, _, _ in derived]
+        self._sources = [(buf, None) for _, bufs, _ in derived for buf in bufs]
 
     def launch(self):
         if not self._handle:
             raise TLError(TL_ERR_INVALID, "graph was destroyed")
+        for buf, version in self._sources:
+            if buf.version != version:
+                if self._ctx.capture is None:
+                    self._bring_up_to_date()
+                break
         check(self._ctx.lib.tl_graph_launch(self._ctx.handle, self._handle))
 
+    def _bring_up_to_date(self):
+        for remake in self._remake:
+            remake()
+        self._sources = [(buf, buf.version) for buf, _ in self._sources]
+
     def destroy(self):
+        self._remake, self._sources = [], []
         if self._handle:
             h, self._handle = self._handle, None
             check(self._ctx.lib.tl_graph_destroy(self._ctx.handle, h))
@@ -1092,18 +1107,20 @@ class capture:  # noqa: N801  (used as a context manager, like torch.cuda.graph)
     def __enter__(self):
         c = ctx()
         check(c.lib.tl_graph_begin(c.handle))
-        c.capturing = True
+        c.capture = self
         self.graph = None
+        self._derived, self._recorded = {}, {}  # copies that the calls read, and that they make
         return self
 
     def __exit__(self, exc_type, exc, tb):
         c = ctx()
         h = ctypes.c_void_p()
-        c.capturing = False
+        c.capture = None
+        derived, self._derived, self._recorded = self._derived.values(), None, None
         rc = c.lib.tl_graph_end(c.handle, ctypes.byref(h))
         if exc_type is None:
             check(rc)
-            self.graph = Graph(h.value)
+            self.graph = Graph(h.value, derived)
         elif rc == TL_OK:
             c.lib.tl_graph_destroy(c.handle, h.value)
         return False
@@ -1118,7 +1135,31 @@ class capture:  # noqa: N801  (used as a context manager, like torch.cuda.graph)
 
 def capturing() -> bool:
     """Whether the context stream is being captured into a graph."""
-    return ctx().capturing
+    return ctx().capture is not None
+
+
+def derived(slots, name, key, sources, make, remake):
+    """make(out), a device tensor made from the tensors `sources` (a packed weight), kept in the
+    dict `slots` under `name` until `key`, the versions it was made from, changes. It is then made
+    again in place: its address stays, and its earlier readers come first on the stream.
+
+    A capture that finds it current records its address: the graph keeps it, and has it made again
+    (`remake`, this call once more) before a launch when a source has been written since.
+    Otherwise the capture records the making, so every replay makes it from the sources as they
+    then are, in a tensor of the graph's own."""
+    cap = (_ctx or ctx()).capture
+    kept = slots.get(name)
+    if cap is None:
+        if kept is None or kept[0] != key:
+            kept = slots[name] = (key, make(kept[1] if kept is not None else None))
+        return kept[1]
+    at = (id(slots), name)
+    if kept is not None and kept[0] == key:
+        cap._derived.setdefault(at, (remake, [t.buf for t in sources], slots))
+        return kept[1]
+    if (at, key) not in cap._recorded:
+        cap._recorded[at, key] = (make(None), slots)
+    return cap._recorded[at, key][0]
 
 
 def attention_supported(dtype, head_dim, kv_capacity) -> bool:
