@@ -86,7 +86,8 @@ enum tl_gemm_tile {
   TL_TILE_PERSIST_256x128_W8 = 12,
   TL_TILE_PERSIST_128x128 = 13,
   /* weight streaming for M <= 16 (decode steps): 16 rows of B per workgroup, K split over
-   * its waves; chosen by TL_TILE_AUTO for M <= 16 up to 32767 columns */
+   * its waves; chosen by TL_TILE_AUTO for M <= 16, but for unbatched products over 32768 or
+   * more columns with no row scaling, K % 64 == 0 and K <= 768, or M >= 4 and K % 2048 != 0 */
   TL_TILE_SKINNY = 14,
   TL_TILE_DMA_256x256_W8 = 15, /* direct global->LDS, 8 waves of 128x64, 2 stages */
   TL_TILE_DMA_128x96 = 16,     /* direct global->LDS, 4 waves of 64x48, 2 stages */

@@ -331,3 +331,19 @@ def test_graphs_keep_and_remake_the_copies_they_read(monkeypatch):
     graph.launch()
     assert made[-1] is kept and copy() is kept
     graph.destroy()
+
+
+@needs_lib
+def test_few_row_products_of_long_k_keep_the_weight_stream():
+    """Up to 16 rows over a wide weight: the streaming kernels where they are the faster ones (K a
+    multiple of 2048; one to three rows on K beyond 768), gemm_rows_kernel elsewhere."""
+    class Rows(ctypes.Structure):
+        _fields_ = [("tile", ctypes.c_int), ("splits", ctypes.c_int), ("us", ctypes.c_float)]
+
+    plan = getattr(ctypes.CDLL(LIB), "_ZN2tl14gemm_rows_planEllli")
+    plan.restype, plan.argtypes = Rows, [ctypes.c_int64] * 3 + [ctypes.c_int]
+    for M, N, K, here in ((4, 50257, 2048, False), (1, 256000, 2048, False), (16, 32768, 4096, False),
+                          (2, 50257, 1024, False), (3, 256000, 1536, False), (16, 32767, 256, False),
+                          (1, 50257, 768, True), (4, 50257, 1024, True), (16, 256000, 1024, True),
+                          (17, 50257, 2048, True)):
+        assert (plan(M, N, K, 256).tile >= 0) == here, (M, N, K)

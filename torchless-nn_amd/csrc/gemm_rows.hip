@@ -268,9 +268,18 @@ static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int elem, int ntiles,
 
 RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
   // M <= 16: the weight-streaming kernels of gemm.hip start faster (3 to 30% on K <= 2048), but
-  // read less of a wide weight at a time: 4 x 50257 x 768 21.5 us against 18.2 here, 4 x 256000
-  // x 2048 212 against 178, 4 x 32768 x 2048 34.4 against 32.5, 4 x 8192 x 1024 equal.
-  if (M <= 16) return N >= 32768 ? rows_best(M, N, K, 2, kNumRowsTiles, cus) : RowsPlan();
+  // gemm_skinny_kernel loads and multiplies the activation rows again for every 16 columns, which
+  // costs more the more rows there are. Over 32768 to 256000 columns with weights that come from
+  // HBM (us, there / here): 1 x 50257 x 256 12.9 / 8.6, 4 x 50257 x 768 19.5 / 17.4, 16 x 50257 x 768
+  // 25.1 / 18.3, 4 x 256000 x 1024 98.9 / 93.3, 16 x 256000 x 1024 143 / 99; but 1 x 256000 x 1024 85.3 /
+  // 89.4, 1 x 50257 x 1536 28.6 / 31.7. On K > 768 four rows break even over seven widths (0.93 to 1.09).
+  // gemm_skinny_stream_kernel (K % 2048 == 0) keeps the rows in registers and stays ahead: 4 x
+  // 50257 x 2048 40.4 / 44.9, 4 x 65536 x 2048 49 / 59, 4 x 256000 x 2048 173 / 178, 16 x 32768 x 2048
+  // 28 / 31, 4 x 65536 x 4096 102 / 110 (K = 4096 beyond 150000 columns: 227 / 216).
+  if (M <= 16) {
+    const bool here = N >= 32768 && K % 2048 != 0 && (K <= 768 || M >= 4);
+    return here ? rows_best(M, N, K, 2, kNumRowsTiles, cus) : RowsPlan();
+  }
   // Products that fill the chip on the tiles of gemm.hip stay there (at 2331 x 2304 x 768 14.9
   // us against 18.8 here), with two exceptions. M <= 64, or <= 128 over many columns, is a
   // stream of the weights, and 256-row tiles only load padding with it (48 x 32768 x 2048 42.4
