@@ -285,7 +285,10 @@ def attention_exact(q, k, vt, causal, offset, Tk):
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("case", [(1, 4, 2, 65, 97, 104, True, 32), (2, 2, 2, 130, 130, 136, False, 0),
                                   (1, 4, 1, 1, 300, 304, True, 299), (3, 2, 1, 33, 129, 136, True, 96),
-                                  (1, 2, 2, 97, 193, 200, False, 0), (2, 3, 3, 321, 321, 328, True, 0)])
+                                  (1, 2, 2, 97, 193, 200, False, 0), (2, 3, 3, 321, 321, 328, True, 0),
+                                  # head dim 32 without pairs of row blocks, below and beyond its lines
+                                  (2, 2, 2, 225, 225, 232, False, 0), (3, 2, 1, 33, 257, 264, True, 224),
+                                  (65, 4, 4, 64, 161, 168, True, 97), (64, 4, 4, 64, 161, 168, True, 97)])
 def test_fp32_attention_pieces(xp, D, case):
     """Row blocks and key halves with remainders, grouped heads, a cache whose padding holds NaN,
     masked halves. Probabilities sum to 1, so errors are a few fp32 ulps of the values."""
@@ -354,7 +357,7 @@ def test_fp32_attention_pieces_tiny_probabilities(xp, D):
     """Values that are huge where the probabilities are tiny and 0 at the key that takes them all;
     scores of up to 124 in log2 units carry 2^-17 of themselves into such a probability. And values
     that are all tiny: outputs within fp32's denormal steps."""
-    B, H, T = 1, 2, 144
+    B, H, T = 1, 2, 240
     rng = np.random.default_rng(D)
     q, k = (rng.standard_normal((B, H, T, D), dtype=F32) * F32(0.05) for _ in range(2))
     vt = np.ldexp(rng.standard_normal((B, H, D, T), dtype=F32), 122)

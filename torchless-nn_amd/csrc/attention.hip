@@ -1782,10 +1782,16 @@ static int attention_fwd(tl_ctx* ctx, const void* q, const void* k, const void* 
   if (dtype == TL_F32) {
     const int64_t nqb = (seq_q + 63) / 64;
     // bf16 pieces on the bf16 matrix cores beyond 96 keys; for fewer the fp32 MFMA's shorter set-up
-    // is as fast or faster (us, fp32 / pieces: T = 17 7.0 / 10.5, 64 9.3 / 10.9, 65 32.2 / 34.4,
-    // 80 15.1 / 12.9, 96 14.9 / 12.7 and 18.9 / 19.5, 128 11.6 / 9.2, 150 29 / 25, 261 69 / 48,
-    // 1000 110 / 63, 1 query on 900 keys 87 / 57)
-    if (head_dim <= 64 && seq_k > 96 && nqb * batch * n_heads_q < (1LL << 31)) {
+    // is as fast or faster (head dim 64, us, fp32 / pieces: T = 17 7.0 / 10.5, 64 9.3 / 10.9, 65 32.2 /
+    // 34.4, 80 15.1 / 12.9, 96 14.9 / 12.7 and 18.9 / 19.5, 128 11.6 / 9.2, 150 29 / 25, 261 69 / 48, 1000
+    // 110 / 63, 1 query on 900 keys 87 / 57). At head dim 32 a workgroup's products are half as long
+    // beside the same set-up, so without the causal kernel's pairs of row blocks the line lies
+    // higher, where the grid leaves CUs without a second workgroup highest (12 heads of 150 without
+    // mask 8.0 / 8.8, of 200 9.7 / 10.0, of 261 11.7 / 11.4, 240 of 192 16.8 / 14.6; 1 query on 97 keys
+    // 6.5 / 7.3, on 256 10.1 / 9.3; causal, 12 heads of 97 9.4 / 7.2).
+    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int64_t keys32 = causal && seq_q > 64 ? 96 : nqb * batch * n_heads_q > cus ? 160 : 224;
+    if (head_dim <= 64 && seq_k > (head_dim == 32 ? keys32 : 96) && nqb * batch * n_heads_q < (1LL << 31)) {
       const int n_bh = (int)(batch * n_heads_q);
       const dim3 g((unsigned)(nqb * n_bh));
       if (head_dim == 32) attention_fwd_pieces_kernel<32><<<g, 256, 0, ctx->stream>>>(p, n_bh);
@@ -1843,7 +1849,11 @@ static int attention_fwd(tl_ctx* ctx, const void* q, const void* k, const void* 
     // workgroups per CU the live blocks are shared out over 4 per CU (us, 96 x 300 of 4096 keys,
     // head dim 256: 118 -> 20; 96 x 3000 of 4096: 119 -> 98; 90 x 2 x 200 of 4096, head dim 128:
     // 111 -> 17; at 6 per CU with most keys live, 48 x 1500 of 2048, 40.4 against 39.9, 24 x 2 x
-    // 1500 of 2048 23.1 against 22.7). With a host position every block is live, and one
+    // 1500 of 2048 23.1 against 22.7). A cache that is full to the end pays for the wait and for one
+    // block after another: over 40 batches and capacities at head dims 32 / 64 / 128 it takes 8%, 2%
+    // and 7% longer on average (96 x 2 x 1024 of 1024 30.2 against 34.7), where 2% to 70% of the
+    // capacity take 33%, 40% and 44% less; 8 workgroups per CU, or the next block's loads ahead of
+    // the merge, move either by 2 to 3%. With a host position every block is live, and one
     // workgroup each is the faster form (24 x 12 x 902 keys, head dim 64: 23.5 against 25.3).
     const int64_t per_round = 4LL * (ctx->num_cus > 0 ? ctx->num_cus : 256);
     w.trim = pos_dev && batch * n_heads_kv * w.nblk > 2 * per_round;
