@@ -91,12 +91,57 @@ def test_few_tiles(xp, dt, mnk):
         assert err <= bar(dt, K), (dt, mnk, kind, err)
 
 
+# Every tile of gemm_rows_kernel (by its number in the tile table: ring depth and K slices per stage
+# 4 x 4, 3 x 2, 5 x 1, 4 x 1, 3 x 1, 2 x 1) at one stage, one short of the ring, the ring and more than
+# twice the ring, whole and in K parts (even, a short last part, an empty last part).
+# dtype, tile, stages, parts, (M, N, K)
+RINGS = [("bf16", 0, 1, 1, (17, 33, 64)), ("bf16", 0, 3, 1, (17, 33, 576)), ("bf16", 0, 4, 1, (17, 33, 832)),
+         ("bf16", 0, 9, 1, (33, 1500, 2112)), ("bf16", 0, 16, 3, (17, 2052, 12288)),
+         ("bf16", 0, 9, 3, (17, 2052, 6208)), ("bf16", 0, 1, 8, (17, 33, 1600)),
+         ("bf16", 1, 1, 1, (17, 8200, 64)), ("bf16", 1, 2, 1, (17, 8200, 192)), ("bf16", 1, 3, 1, (17, 8200, 320)),
+         ("bf16", 1, 7, 1, (17, 8200, 832)), ("bf16", 1, 7, 5, (17, 3000, 4160)), ("bf16", 1, 11, 3, (17, 4100, 4160)),
+         ("bf16", 2, 1, 1, (33, 33, 64)), ("bf16", 2, 4, 1, (33, 8200, 256)), ("bf16", 2, 5, 1, (33, 4100, 320)),
+         ("bf16", 2, 11, 1, (33, 4100, 704)), ("bf16", 2, 12, 16, (513, 33, 12288)),
+         ("bf16", 2, 11, 6, (65, 1000, 4160)), ("bf16", 2, 9, 16, (700, 33, 8320)), ("bf16", 2, 32, 8, (48, 2048, 16384)),
+         ("bf16", 3, 1, 1, (1, 32776, 64)), ("bf16", 3, 3, 1, (1, 32776, 192)), ("bf16", 3, 4, 1, (1, 32776, 256)),
+         ("bf16", 3, 9, 1, (1, 32776, 576)), ("bf16", 3, 10, 5, (18, 8200, 3200)), ("bf16", 3, 9, 12, (17, 4100, 6208)),
+         ("bf16", 4, 1, 1, (33, 32776, 64)), ("bf16", 4, 2, 1, (33, 32776, 128)), ("bf16", 4, 3, 1, (33, 32776, 192)),
+         ("bf16", 4, 7, 1, (33, 32776, 448)), ("bf16", 4, 17, 3, (33, 16400, 3136)),
+         ("bf16", 5, 1, 1, (65, 50257, 64)), ("bf16", 5, 2, 1, (65, 50257, 128)), ("bf16", 5, 3, 1, (65, 50257, 192)),
+         ("bf16", 5, 5, 1, (65, 50257, 320)), ("bf16", 5, 17, 6, (65, 8200, 6208)),
+         ("fp32", 0, 1, 1, (1, 33, 32)), ("fp32", 0, 3, 1, (1, 33, 288)), ("fp32", 0, 4, 1, (1, 2052, 416)),
+         ("fp32", 0, 9, 1, (16, 6000, 1056)), ("fp32", 0, 16, 3, (129, 516, 6144)), ("fp32", 0, 11, 6, (1, 1025, 8192)),
+         ("fp32", 0, 2, 16, (1, 33, 3104)), ("fp32", 1, 1, 1, (1, 8200, 32)), ("fp32", 1, 2, 1, (1, 8200, 96)),
+         ("fp32", 1, 3, 1, (1, 8200, 160)), ("fp32", 1, 7, 1, (1, 12000, 416)), ("fp32", 1, 8, 16, (1, 1500, 8192)),
+         ("fp32", 1, 7, 3, (1, 8200, 1280)), ("fp32", 1, 3, 12, (1, 2052, 2048)), ("fp32", 2, 1, 1, (33, 33, 32)),
+         ("fp32", 2, 4, 1, (33, 8200, 128)), ("fp32", 2, 5, 1, (33, 8200, 160)), ("fp32", 2, 11, 1, (33, 8200, 352)),
+         ("fp32", 2, 16, 16, (513, 33, 8192)), ("fp32", 2, 11, 12, (33, 1025, 4096)), ("fp32", 2, 6, 12, (33, 1025, 2048))]
+
+
+@pytest.mark.parametrize("dt,tile,stages,parts,mnk", RINGS)
+def test_few_tiles_rings(xp, dt, tile, stages, parts, mnk):
+    M, N, K = mnk
+    assert plan(xp, dt, M, N, K) == ("rows", tile, parts)
+    per_part = -(-(K // (64 if dt == "bf16" else 32)) // parts)
+    assert -(-per_part // (4, 2, 1, 1, 1, 1)[tile]) == stages
+    a, w, bias, res = inputs(xp, dt, M, N, K)
+    out = xp.empty((M, N), dt, pitch=(N + 7) // 8 * 8)
+    xp.gemm(xp.array(a, dtype=dt), xp.array(w, dtype=dt), M=M, N=N, K=K, lda=K, ldb=K, b_layout=xp.TL_B_NK,
+            C=out, ldc=out.pitch, bias=xp.array(bias, dtype=dt), residual=xp.array(res, dtype=dt), ldr=N)
+    want = a.astype(np.float64) @ w.astype(np.float64).T + bias + res
+    assert ref.max_rel(out.get(), want) <= bar(dt, K)
+
+
 @pytest.mark.parametrize("dt", ["fp32", "bf16"])
 @pytest.mark.parametrize("cfg", [(24, 1, 4, 4, 64, 40, 37, 256), (3, 21, 8, 2, 32, 64, 5, 2048),
-                                 (40, 7, 4, 1, 64, 16, 8, 128), (5, 300, 2, 2, 64, 304, 0, 128)])
+                                 (40, 7, 4, 1, 64, 16, 8, 128), (5, 300, 2, 2, 64, 304, 0, 128),
+                                 (5, 401, 8, 2, 64, 416, 7, 2048), (6, 11, 24, 24, 128, 16, 1, 832),
+                                 (66, 1, 64, 64, 256, 8, 0, 192), (4, 500, 8, 8, 64, 512, 3, 256),
+                                 (4, 1000, 12, 12, 64, 1008, 0, 768)])
 def test_few_tiles_head_scatter(xp, dt, cfg):
     """The QKV scatter into q and a cache at an odd position (one new position per sequence,
-    short odd prompts), with and without parts of K; untouched cache rows stay."""
+    short odd prompts), with and without parts of K, and over the larger tiles of both kernels;
+    untouched cache rows stay."""
     B, T, Hq, Hkv, D, L, pos0, K = cfg
     M, N = B * T, (Hq + 2 * Hkv) * D
     a, w, bias, _ = inputs(xp, dt, M, N, K)
@@ -113,16 +158,18 @@ def test_few_tiles_head_scatter(xp, dt, cfg):
         assert ref.max_rel(got.get(), want) <= bar(dt, K), cfg
 
 
-@pytest.mark.parametrize("mnk", [(24, 512, 512), (48, 1000, 4096), (100, 200, 128), (17, 66000, 64)])
-def test_few_tiles_gated(xp, mnk):
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
+@pytest.mark.parametrize("mnk", [(24, 512, 512), (48, 1000, 4096), (100, 200, 128), (17, 66000, 64), (17, 8200, 320),
+                                 (33, 16400, 3136), (65, 1000, 4160), (1281, 1538, 1024)])
+def test_few_tiles_gated(xp, mnk, dt):
     M, N, K = mnk
-    a, w, _, _ = inputs(xp, "bf16", M, N, K)
-    out = xp.empty((M, N // 2), "bf16")
-    xp.gemm(xp.array(a, dtype="bf16"), xp.array(w, dtype="bf16"), M=M, N=N, K=K, lda=K, ldb=K,
+    a, w, _, _ = inputs(xp, dt, M, N, K)
+    out = xp.empty((M, N // 2), dt)
+    xp.gemm(xp.array(a, dtype=dt), xp.array(w, dtype=dt), M=M, N=N, K=K, lda=K, ldb=K,
             b_layout=xp.TL_B_NK, C=out, ldc=N // 2, act=xp.TL_ACT_SILU, geglu=True)
     y = a.astype(np.float64) @ w.astype(np.float64).T
     want = ref.silu(y[:, 0::2]).astype(np.float64) * y[:, 1::2]
-    assert ref.max_rel(out.get(), want) <= bar("bf16", K)
+    assert ref.max_rel(out.get(), want) <= bar(dt, K)
 
 
 # whole tiles only, a last round split over K, everything split, tails of one row and column,
@@ -445,3 +492,22 @@ def test_decode_trims_dead_blocks(xp, D, Hkv, pos):
     got = dk.get()
     assert np.array_equal(np.isnan(got), np.isnan(k))
     assert ref.max_rel(np.nan_to_num(got), np.nan_to_num(k)) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,Tq,L,pos", [(32, 8, 8, 1, 512, 0), (32, 8, 8, 2, 512, 300), (32, 4, 2, 3, 1024, 1021),
+                                              (64, 8, 2, 2, 1024, 126), (128, 4, 2, 4, 1024, 700),
+                                              (256, 8, 1, 2, 1024, 1022), (64, 8, 4, 1, 512, 512), (32, 8, 8, 2, 512, 511)])
+def test_decode_trims_several_positions(xp, D, Hq, Hkv, Tq, L, pos):
+    """The trimmed grid with one to four query positions, at head dim 32 too, up to the last key and
+    at a position that the capacity cuts off (rows past it see the keys that there are)."""
+    B = -(-2100 * 64 // (Hkv * L))
+    rng = np.random.default_rng(pos + D)
+    q = ref.round_bf16(rng.standard_normal((B, Hq, Tq, D), dtype=F32))
+    k, vt = (ref.round_bf16(rng.standard_normal(s, dtype=F32)) for s in ((B, Hkv, L, D), (B, Hkv, D, L)))
+    k[:, :, pos + Tq:], vt[..., pos + Tq:] = np.nan, np.nan
+    out = xp.empty((B, Tq, Hq * D), "bf16")
+    xp.attention_decode_dev(*(xp.array(t, dtype="bf16") for t in (q, k, vt)), out,
+                            xp.array(np.array([pos], np.int64)), n_heads_q=Hq, n_heads_kv=Hkv,
+                            divisor=float(F32(D ** 0.5)))
+    want = attention_exact(q, k, vt, True, pos, min(pos + Tq, L))
+    assert ref.max_rel(out.get(), want) <= 2e-2
