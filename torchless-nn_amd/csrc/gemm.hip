@@ -15,7 +15,10 @@
 //   run of tiles, and tiles run in groups of a few tile-rows (group_m) so the A and B panels
 //   a group shares stay in that XCD's L2.
 // gemm_simt_kernel: any dtype, layout or alignment, fp32 FMA on the vector ALUs. It
-//   serves the fp32 model and shapes the MFMA kernel's 16-byte loads cannot take.
+//   serves shapes that the MFMA kernels' 16-byte loads cannot take, and few fp32 tiles with
+//   K % 32 != 0.
+// Products with few output tiles, most fp32 products and 256x256 tiles that fill the chip run in
+// gemm_rows.hip, gemm_split.hip and gemm_pp.hip; tl_gemm below chooses.
 #include <algorithm>
 
 #include "gemm_epilogue.hpp"
@@ -1194,17 +1197,17 @@ extern "C" int tl_gemm(tl_ctx* ctx, const tl_gemm_desc* d) {
   const double flops = 2.0 * d->M * d->N * d->K * batch;
   const double bytes = batch * (es_in * ((double)d->M * d->K + (double)d->N * d->K) +
                                 (double)eo * d->M * d->N * (d->residual ? 2 : 1));
-  // fp32 operands on the matrix cores under the same layout rules (4-element alignment) when
-  // there are at least 128 output tiles of 128x128; fewer stay on the split-K VALU kernel.
+  // fp32 operands on the matrix cores under the same layout rules (4-element alignment): unbatched
+  // with K % 32 == 0 in gemm_rows.hip or gemm_split.hip (below), otherwise here when there are at
+  // least 128 output tiles of 128x128; fewer stay on the split-K VALU kernel.
   const bool mfma32_layout = d->dtype_in == TL_F32 && d->b_layout == TL_B_NK && d->K % 4 == 0 &&
                              d->lda % 4 == 0 && d->ldb % 4 == 0 && d->sa_o % 4 == 0 &&
                              d->sa_i % 4 == 0 && d->sb_o % 4 == 0 && d->sb_i % 4 == 0 &&
                              al16(d->A) && al16(d->B) && d->lda * 128 < (1LL << 31) &&
                              d->ldb * 128 < (1LL << 31);
   const bool mfma32 = mfma32_layout && ((d->M + 127) / 128) * ((d->N + 127) / 128) * batch >= 128;
-  // small fp32 products with a short K loop (the char-level GPT: M = 512, K = 128 .. 512)
-  // on 64x64 fp32 MFMA tiles rather than the vector ALUs; long K with few tiles stays on the
-  // split-K vector kernel
+  // of those, small products with a short K loop on 64x64 fp32 MFMA tiles rather than the vector
+  // ALUs; long K with few tiles stays on the split-K vector kernel
   const bool mfma32_small = mfma32_layout && !mfma32 && d->K <= 1024 &&
                             ((d->M + 63) / 64) * ((d->N + 63) / 64) * batch >= 8;
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;

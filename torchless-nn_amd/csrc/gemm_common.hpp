@@ -188,7 +188,7 @@ __device__ __forceinline__ void epilogue4(const GemmParams& p, int64_t zo, int64
   }
 }
 
-// The kernel's only argument is a GemmParams by value, at offset 0 of the kernarg segment.
+// For kernels whose first argument is a GemmParams by value, at offset 0 of the kernarg segment.
 // The epilogue re-reads it through an opaque copy of the segment pointer: those loads
 // cannot be hoisted to the kernel entry, so the ~40 scalar registers of epilogue fields
 // are not held across the K loop (holding them made the large tiles spill to scratch).

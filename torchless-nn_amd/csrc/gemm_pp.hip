@@ -15,8 +15,8 @@
 //
 // us against the tiles used before: 8192^3 801 -> 757 (1453 TFLOP/s), 8192 x 32768 x 2048 (gated)
 // 846 -> 794, 8192 x 2048 x 2048 78 -> 64, 8192 x 4096 x 1024 80 -> 64, 8192 x 6144 x 768 (GeLU)
-// 110 -> 92, 8192 x 50257 x 768 702 -> 672, 8192 x 2048 x 16384 441 -> 433. What bounds it is the
-// LDS: with the loads left out it runs at 2.1 PFLOP/s, with all loads from the same cached lines
+// 110 -> 92, 8192 x 50257 x 768 685 -> 668 (the LM head in the GPT-2 forward, kernel traces in turn),
+// 8192 x 2048 x 16384 441 -> 433. What bounds it is the LDS: with the loads left out it runs at 2.1 PFLOP/s, with all loads from the same cached lines
 // at 1.53, so the 64 KB a step writes into LDS beside the 192 KB it reads costs more than their
 // latency. Tried: loads among the MFMAs instead of the reads (1429 TFLOP/s at 8192^3, 460 us at K =
 // 16384), five 32-wide stages (twice the lookahead, 1314), no s_setprio (1354), a 256x192 tile (ties
