@@ -392,7 +392,11 @@ class DeviceTensor:
 
     def _rows(self):
         """The same rows as a 2-d tensor."""
-        return self._reshaped((self.nrows, self.ncols), self.nrows, self.ncols)
+        t = object.__new__(DeviceTensor)
+        t.nrows, t.ncols = t.shape = self.nrows, self.ncols
+        t.dtype, t.buf, t.offset, t.ptr = self.dtype, self.buf, self.offset, self.ptr
+        t.size, t.pitch, t._aux = self.size, self.pitch, None
+        return t
 
     def _reshaped(self, shape, nrows, ncols):
         """The same elements under `shape`, a tuple of ints with `nrows` rows of `ncols` (rows of
