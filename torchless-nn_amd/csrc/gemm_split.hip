@@ -18,8 +18,9 @@
 // by row / 2, so that the writes and the fragment reads meet no bank conflicts). Two forms: 256x128
 // with 8 waves of 64x64 and two LDS buffers, where a step's splitting (132 vector instructions per
 // wave) is scheduled among the 96 MFMAs of the step before it, and 128x64 with 4 waves of 64x32 and
-// one buffer, three workgroups per CU, whose phases overlap each other's. Bound by the matrix cores
-// and the LDS reads (24 fragments per 96 MFMAs) once the chip is full: 8192 x 50257 x 768 5801 ->
+// one buffer, three workgroups per CU, whose phases overlap each other's. Once the chip is full the
+// matrix cores are busy 0.42 to 0.46 of the time and each of the two waves per SIMD issues vector
+// instructions for 0.22 of it; neither alone bounds it: 8192 x 50257 x 768 5801 ->
 // 3262 us (194 TFLOP/s of fp32 products, 1.16 PFLOP/s on the matrix cores), 4000 x 3072 x 768 174 ->
 // 107, 4000 x 768 x 3072 230 -> 108 us; error against 64 bits 4.2e-7 where the fp32 MFMA's is
 // 5.0e-7 (1024 x 50257 x 768; 0.78 to 0.85 of it over 10007 to 50257 columns, K 256 .. 768). The
