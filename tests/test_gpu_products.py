@@ -315,6 +315,52 @@ def test_parts_without_workspace(dt, mnk):
         xp._ctx = old
 
 
+# M, N, K, and the kernel that takes it in fp32 and in bf16 (None: the tiles of gemm.hip, or gemm_pp_kernel)
+ODD_FORMS = [(21, 131, 576, "rows", "rows"), (65, 258, 4096, "rows", "rows"), (1029, 770, 1024, "rows", "rows"),
+             (2051, 1030, 256, "split", "rows"), (1281, 769, 3072, "split", "rows"), (2050, 8197, 320, "split", None)]
+
+
+@pytest.mark.parametrize("out_dt", ["fp32", "bf16"])
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
+@pytest.mark.parametrize("M,N,K,k32,k16", ODD_FORMS)
+def test_odd_operand_forms(xp, M, N, K, k32, k16, dt, out_dt):
+    """Rows apart by more than their length and operands that start inside a buffer (16 bytes in, the
+    least that the matrix-core kernels take), outputs and residuals at odd offsets and pitches, a
+    divisor, either type in and out, the residual overwritten by the result; nothing outside the
+    output's rows is written."""
+    got = plan(xp, dt, M, N, K)
+    assert (got and got[0]) == (k32 if dt == "fp32" else k16)
+    a, w, bias, res = inputs(xp, dt, M, N, K)
+    if out_dt == "bf16":
+        res = ref.round_bf16(res)
+    y = a.astype(np.float64) @ w.astype(np.float64).T
+
+    def strided(host, dtype, pitch, first):
+        rows, cols = host.shape
+        flat = np.full(first + rows * pitch, 7, F32)
+        flat[first:].reshape(rows, pitch)[:, :cols] = host
+        t = xp.array(flat, dtype=dtype)
+        return t, xp.DeviceTensor((1,), dtype, buf=t.buf, offset=first * t.dtype.itemsize)
+
+    step = 4 if dt == "fp32" else 8
+    _, da = strided(a, dt, K + 2 * step, step)
+    _, dw = strided(w, dt, K + 3 * step, step)
+    db = xp.array(np.r_[F32(9), bias], dtype=dt)
+    bias_at = xp.DeviceTensor((N,), dt, buf=db.buf, offset=db.dtype.itemsize)
+    tol = 2 * bar(out_dt, K)  # the activation and the residual add their own roundings
+    for pitch, first, in_place in ((N + 3, 1, False), (N + 1, 3, True), ((N + 11) // 8 * 8, 8, False)):
+        whole, out = strided(res if in_place else np.zeros_like(res), out_dt, pitch, first)
+        _, dres = strided(res, out_dt, N + 5, 3)
+        xp.gemm(da, dw, M=M, N=N, K=K, lda=K + 2 * step, ldb=K + 3 * step, b_layout=xp.TL_B_NK, C=out, ldc=pitch,
+                out_dtype=out_dt, bias=bias_at, act=xp.TL_ACT_SILU, divisor=2.0,
+                residual=out if in_place else dres, ldr=pitch if in_place else N + 5)
+        flat = whole.get()
+        rows = flat[first:].reshape(M, pitch)
+        want = ref.silu(y / 2 + bias).astype(np.float64) + res
+        assert ref.max_rel(rows[:, :N], want) <= tol, (pitch, first)
+        assert np.all(flat[:first] == 7) and np.all(rows[:, N:] == 7), (pitch, first)
+
+
 def attention_exact(q, k, vt, causal, offset, Tk):
     """float64 attention of q [B, H, T, D] over the first Tk keys, heads merged [B, T, H D]."""
     q, k, v = (t.astype(np.float64) for t in (q, k[:, :, :Tk], np.swapaxes(vt[..., :Tk], 2, 3)))
