@@ -202,8 +202,8 @@ int tl_prefetch_hint(tl_ctx* ctx, const void* ptr, int64_t bytes);
  * tl_graph_end, which instantiates them. While a capture is open, calls that wait for the
  * stream (tl_sync, host copies) fail with TL_ERR_INVALID, the kernel profiler records
  * nothing, and a call that cannot do without a workspace that would have to grow fails (run
- * the step once before capturing it). tl_gemm for more than 16 rows, or over 32768 or more
- * columns, does without: it then takes all of K per workgroup, so its sums are added in another
+ * the step once before capturing it). On the matrix cores tl_gemm does without for more than 16
+ * rows or 32767 columns: it then takes all of K per workgroup, so its sums are added in another
  * order than in a call with the workspace. Device blocks that tl_malloc hands out during the capture belong to
  * the graph until tl_graph_destroy: replays write them, so they are kept from reuse even
  * after the caller frees them. tl_graph_launch replays the graph on the context stream. */

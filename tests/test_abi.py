@@ -340,10 +340,11 @@ def test_few_row_products_of_long_k_keep_the_weight_stream():
     class Rows(ctypes.Structure):
         _fields_ = [("tile", ctypes.c_int), ("splits", ctypes.c_int), ("us", ctypes.c_float)]
 
-    plan = getattr(ctypes.CDLL(LIB), "_ZN2tl14gemm_rows_planEllli")
-    plan.restype, plan.argtypes = Rows, [ctypes.c_int64] * 3 + [ctypes.c_int]
+    plan = getattr(ctypes.CDLL(LIB), "_ZN2tl14gemm_rows_planElllib")
+    plan.restype, plan.argtypes = Rows, [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.c_bool]
     for M, N, K, here in ((4, 50257, 2048, False), (1, 256000, 2048, False), (16, 32768, 4096, False),
                           (2, 50257, 1024, False), (3, 256000, 1536, False), (16, 32767, 256, False),
                           (1, 50257, 768, True), (4, 50257, 1024, True), (16, 256000, 1024, True),
                           (17, 50257, 2048, True)):
-        assert (plan(M, N, K, 256).tile >= 0) == here, (M, N, K)
+        assert (plan(M, N, K, 256, True).tile >= 0) == here, (M, N, K)
+    assert plan(4, 50257, 4096, 256, False).tile >= 0  # without workspace for the stream's K parts

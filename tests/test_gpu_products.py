@@ -35,12 +35,12 @@ class _Split(ctypes.Structure):
 def plan(xp, dt, M, N, K, cus=256):
     """What tl_gemm makes of an unbatched [M, K] x [N, K] product with a plain tile hint: ("rows",
     tile, splits), ("split", tile, whole tiles, splits), or None for the other kernels."""
-    def call(symbol, result):
+    def call(symbol, result, *more):
         f = getattr(xp.load_library(), symbol)
-        f.restype, f.argtypes = result, [ctypes.c_int64] * 3 + [ctypes.c_int]
-        return f(M, N, K, cus)
+        f.restype, f.argtypes = result, [ctypes.c_int64] * 3 + [ctypes.c_int] + [ctypes.c_bool] * len(more)
+        return f(M, N, K, cus, *more)
     if dt == "bf16":
-        r = call("_ZN2tl14gemm_rows_planEllli", _Rows)
+        r = call("_ZN2tl14gemm_rows_planElllib", _Rows, True)
         return ("rows", r.tile, r.splits) if r.tile >= 0 else None
     r, s = call("_ZN2tl18gemm_rows_plan_f32Ellli", _Rows), call("_ZN2tl15gemm_split_planEllli", _Split)
     if r.tile >= 0 and (s.tile < 0 or r.us <= s.us):
@@ -286,7 +286,7 @@ def test_fp32_pieces_not_finite(xp, mnk):
 
 
 @pytest.mark.parametrize("dt,mnk", [("bf16", (24, 768, 3072)), ("fp32", (24, 768, 3072)),
-                                    ("fp32", (1281, 769, 3072))])
+                                    ("fp32", (1281, 769, 3072)), ("bf16", (4, 32776, 4096))])
 def test_parts_without_workspace(dt, mnk):
     """A fresh context whose first product is captured: the workspace cannot grow then, so the
     product takes one workgroup per tile; replays and a later eager call agree."""

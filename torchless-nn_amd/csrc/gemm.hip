@@ -1217,7 +1217,9 @@ extern "C" int tl_gemm(tl_ctx* ctx, const tl_gemm_desc* d) {
   RowsPlan rows;
   SplitPlan split32;
   if (d->tile == TL_TILE_AUTO && batch == 1 && !d->norm_rows && d->lda < (1 << 24) && d->ldb < (1 << 24)) {
-    if (mfma && d->K % 64 == 0) rows = gemm_rows_plan(d->M, d->N, d->K, cus);
+    const size_t stream_ws = d->K > 2048 ? (size_t)((d->N + 15) / 16 * (d->K / 2048)) * 1024 : 0;
+    const bool can_stream = !ctx->capturing || stream_ws <= ctx->ws_bytes;  // a capture cannot grow it
+    if (mfma && d->K % 64 == 0) rows = gemm_rows_plan(d->M, d->N, d->K, cus, can_stream);
     if (mfma32_layout && d->K % 32 == 0) {
       rows = gemm_rows_plan_f32(d->M, d->N, d->K, cus);
       split32 = gemm_split_plan(d->M, d->N, d->K, cus);

@@ -266,7 +266,7 @@ static RowsPlan rows_best(int64_t M, int64_t N, int64_t K, int elem, int ntiles,
   return best;
 }
 
-RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
+RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus, bool can_stream) {
   // M <= 16: the weight-streaming kernels of gemm.hip start faster (3 to 30% on K <= 2048), but
   // gemm_skinny_kernel loads and multiplies the activation rows again for every 16 columns, which
   // costs more the more rows there are. Over 32768 to 256000 columns with weights that come from
@@ -275,9 +275,10 @@ RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
   // 89.4, 1 x 50257 x 1536 28.6 / 31.7. On K > 768 four rows break even over seven widths (0.93 to 1.09).
   // gemm_skinny_stream_kernel (K % 2048 == 0) keeps the rows in registers and stays ahead: 4 x
   // 50257 x 2048 40.4 / 44.9, 4 x 65536 x 2048 49 / 59, 4 x 256000 x 2048 173 / 178, 16 x 32768 x 2048
-  // 28 / 31, 4 x 65536 x 4096 102 / 110 (K = 4096 beyond 150000 columns: 227 / 216).
+  // 28 / 31, 4 x 65536 x 4096 102 / 110 (K = 4096 beyond 150000 columns: 227 / 216). Its K parts need
+  // a workspace, which this kernel can do without.
   if (M <= 16) {
-    const bool here = N >= 32768 && K % 2048 != 0 && (K <= 768 || M >= 4);
+    const bool here = N >= 32768 && (K % 2048 == 0 ? !can_stream : K <= 768 || M >= 4);
     return here ? rows_best(M, N, K, 2, kNumRowsTiles, cus) : RowsPlan();
   }
   // Products that fill the chip on the tiles of gemm.hip stay there (at 2331 x 2304 x 768 14.9

@@ -13,7 +13,8 @@ struct RowsPlan {
 };
 // The choice for an unbatched product [M, K] x [N, K] whose K is a multiple of 128 bytes (rules
 // from measurements): bf16 operands, and fp32 ones (whose time competes with SplitPlan's).
-RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus);
+// `can_stream`: whether gemm_skinny_stream_kernel can have its workspace.
+RowsPlan gemm_rows_plan(int64_t M, int64_t N, int64_t K, int cus, bool can_stream);
 RowsPlan gemm_rows_plan_f32(int64_t M, int64_t N, int64_t K, int cus);
 // Runs it. Operands as gemm_mfma_kernel / gemm_mfma_f32_kernel take them, batch 1.
 int gemm_rows_launch(tl_ctx* ctx, GemmParams p, RowsPlan plan, bool f32in, bool f32out, int family,
