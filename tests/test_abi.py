@@ -313,7 +313,7 @@ def test_graphs_keep_and_remake_the_copies_they_read(monkeypatch):
     kept = copy()
     assert kept is not recorded and made == [None, None]
     read, graph = captured()
-    assert read is kept and len(made) == 2
+    assert read is kept and len(made) == 2 and [copy_ for _, copy_ in graph._remake] == [kept]
     graph.launch()
     assert len(made) == 2  # still current
     source._version += 1

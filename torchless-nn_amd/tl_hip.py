@@ -1074,7 +1074,7 @@ class Graph:
         self._handle, self._ctx = handle, ctx()
         # copies that the captured calls read (a packed weight): how each is brought up to date, and
         # the version of every buffer they are made from when that was last done
-        self._remake = [remake for remake, _, _ in derived]
+        self._remake = [(remake, copy) for remake, _, copy in derived]
         self._sources = [(buf, None) for _, bufs, _ in derived for buf in bufs]
 
     def launch(self):
@@ -1088,7 +1088,7 @@ class Graph:
         check(self._ctx.lib.tl_graph_launch(self._ctx.handle, self._handle))
 
     def _bring_up_to_date(self):
-        for remake in self._remake:
+        for remake, _ in self._remake:
             remake()
         self._sources = [(buf, buf.version) for buf, _ in self._sources]
 
@@ -1159,10 +1159,10 @@ def derived(slots, name, key, sources, make, remake):
         return kept[1]
     at = (id(slots), name)
     if kept is not None and kept[0] == key:
-        cap._derived.setdefault(at, (remake, [t.buf for t in sources], slots))
+        cap._derived.setdefault(at, (remake, [t.buf for t in sources], kept[1]))
         return kept[1]
     if (at, key) not in cap._recorded:
-        cap._recorded[at, key] = (make(None), slots)
+        cap._recorded[at, key] = (make(None), slots)  # (`slots` keeps its id from being reused)
     return cap._recorded[at, key][0]
 
 
