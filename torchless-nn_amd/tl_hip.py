@@ -1072,10 +1072,10 @@ class Graph:
 
     def __init__(self, handle, derived=()):
         self._handle, self._ctx = handle, ctx()
-        # copies that the captured calls read (a packed weight): how each is brought up to date, and
-        # the version of every buffer they are made from when that was last done
+        # copies that the captured calls read (a packed weight) and how each is brought up to date;
+        # every buffer they are made from, with its version when they were made
         self._remake = [(remake, copy) for remake, _, copy in derived]
-        self._sources = [(buf, None) for _, bufs, _ in derived for buf in bufs]
+        self._sources = [source for _, sources, _ in derived for source in sources]
 
     def launch(self):
         if not self._handle:
@@ -1159,7 +1159,7 @@ def derived(slots, name, key, sources, make, remake):
         return kept[1]
     at = (id(slots), name)
     if kept is not None and kept[0] == key:
-        cap._derived.setdefault(at, (remake, [t.buf for t in sources], kept[1]))
+        cap._derived.setdefault(at, (remake, [(t.buf, t.buf.version) for t in sources], kept[1]))
         return kept[1]
     if (at, key) not in cap._recorded:
         cap._recorded[at, key] = (make(None), slots)  # (`slots` keeps its id from being reused)
